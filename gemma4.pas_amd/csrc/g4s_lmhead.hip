@@ -155,25 +155,96 @@ __global__ __launch_bounds__(kLmBlock) void lmhead_q4_kernel(const uint8_t* __re
 }
 
 /* ------------------------------------------------------------------
- * TILED64 layout and the LM head over it.
+ * The matrix-core sum of 64 weight rows (lane = row) for 4 * NG hidden
+ * vectors.
  *
- * One wave per 64 weight rows (lane = row), waves independent (no LDS, no
- * barrier).  Per 32-column block a lane loads its row's binary32 scale and
- * 16 nibble bytes from the tile (256 + 1024 contiguous bytes per wave) one
- * block ahead, and dequantises the 32 weights once for the 32 hidden
- * vectors of the batch tile.  The hidden values reach the fma without LDS:
- * a 16-byte load per lane brings two vectors' 32 values of the block into
- * four VGPRs (lanes 0-7 of every 16-lane row: vector b, columns 4n..4n+3;
- * lanes 8-15: vector b+1), and v_fmac_f32 with the DPP modifier
- * row_newbcast:n hands lane n's value of its 16-lane row to all lanes of
- * that row -- the same value in all four rows, so every lane sees it.  Each
- * logit is still one fma per term in column order (the order argument at
- * the top of this file), the 32 vectors being 32 independent chains.
+ * v_mfma_f32_4x4x1_16b multiplies a 4x1 by a 1x4 in each of 16 blocks: one
+ * product per output, so one instruction is one binary32 fma of every chain
+ * and a sequence of them keeps the reference's order (checked bit for bit
+ * against fmaf: ties, denormals, infinities and NaN included).  The weights
+ * are the B operand: block b, column j is lane 4b + j, that is the lane's own
+ * row.  The hidden values are the A operand with CBSZ = 4: block ABID's four
+ * rows (vectors) go to all 16 blocks, so one VGPR holds four vectors' values
+ * of 16 columns and nothing passes through LDS.  D: register i of a lane is
+ * vector i of the lane's row.
+ *
+ * It runs 32 fmas per clock and SIMD (135 TFLOP/s measured, against 66 for
+ * v_fmac_f32 with a DPP broadcast).  The binary32 matrix instructions share
+ * the VALU's issue (a wave of each takes the sum of the two times), so the
+ * dequantisation adds to them: 262,144 rows x 2,560 columns take 38 us of
+ * matrix instructions per four vectors and about 60 us for the rest.
  * ------------------------------------------------------------------ */
 
-constexpr int kTileB = 32;        /* hidden vectors per pass over the weights */
-constexpr int kTileWaves = 4;     /* waves (64-row groups) per workgroup */
-constexpr int kXAhead = 4;        /* vector pairs whose values are in flight */
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+/* Eight weights of a row: nibble t of `w` is weight t.  A byte 0..15 read as
+ * fp8 (e4m3) is n * 2^-9 (its denormals and first binade), so one
+ * v_cvt_pk_f32_fp8 gives two nibbles, and fma(n * 2^-9, 512 s, -8 s) is
+ * (n - 8) s exactly (at most 15 significant bits).  s512 = 512 s, m8 = -8 s. */
+__device__ __forceinline__ void dequant8(uint32_t w, float s512, float m8, float (&q)[8])
+{
+    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+    const auto l0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, false);
+    const auto l1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, true);
+    const auto h0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, false);
+    const auto h1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, true);
+    q[0] = __builtin_fmaf(l0[0], s512, m8);
+    q[1] = __builtin_fmaf(h0[0], s512, m8);
+    q[2] = __builtin_fmaf(l0[1], s512, m8);
+    q[3] = __builtin_fmaf(h0[1], s512, m8);
+    q[4] = __builtin_fmaf(l1[0], s512, m8);
+    q[5] = __builtin_fmaf(h1[0], s512, m8);
+    q[6] = __builtin_fmaf(l1[1], s512, m8);
+    q[7] = __builtin_fmaf(h1[1], s512, m8);
+}
+
+/* Terms 8W .. 8W+7 of a block.  x[g]: lane l holds columns 2 (l / 4) and
+ * 2 (l / 4) + 1 of vector 4g + l % 4. */
+template <int W, int NG>
+__device__ __forceinline__ void mac8(f32x4 (&S)[NG], const float (&q)[8], const float2 (&x)[NG])
+{
+#define G4S_MAC(T, C, AB)                                                                       \
+    _Pragma("unroll") for (int g = 0; g < NG; ++g)                                              \
+        S[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(x[g].C, q[T], S[g], 4, AB, 0);
+    G4S_MAC(0, x, 4 * W)
+    G4S_MAC(1, y, 4 * W)
+    G4S_MAC(2, x, 4 * W + 1)
+    G4S_MAC(3, y, 4 * W + 1)
+    G4S_MAC(4, x, 4 * W + 2)
+    G4S_MAC(5, y, 4 * W + 2)
+    G4S_MAC(6, x, 4 * W + 3)
+    G4S_MAC(7, y, 4 * W + 3)
+#undef G4S_MAC
+}
+
+/* The 32 terms of one block. */
+template <int NG>
+__device__ __forceinline__ void mac32(f32x4 (&S)[NG], const uint4 w, float sc, const float2 (&x)[NG])
+{
+    const float s512 = 512.0f * sc, m8 = -8.0f * sc;
+    float q[8];
+    dequant8(w.x, s512, m8, q);
+    mac8<0, NG>(S, q, x);
+    dequant8(w.y, s512, m8, q);
+    mac8<1, NG>(S, q, x);
+    dequant8(w.z, s512, m8, q);
+    mac8<2, NG>(S, q, x);
+    dequant8(w.w, s512, m8, q);
+    mac8<3, NG>(S, q, x);
+}
+
+/* ------------------------------------------------------------------
+ * TILED64 layout and the LM head over it.
+ *
+ * One wave per 64 weight rows and 4 * NG hidden vectors, waves independent
+ * (no LDS, no barrier).  Per 32-column block a lane loads its row's binary32
+ * scale and 16 nibble bytes from the tile (256 + 1024 contiguous bytes per
+ * wave) and two columns of its vectors (L1/L2 hits), kept DEPTH blocks ahead
+ * in registers.  262,144 x 2,560 (a plain read of the 419 MB of tiles takes
+ * 69-73 us): B = 1 645 -> 74 us, B = 8 138 us, B = 32 649 -> 366 us.
+ * ------------------------------------------------------------------ */
+
+constexpr int kTileWaves = 4; /* waves (64-row groups) per workgroup */
 
 __global__ __launch_bounds__(256) void q4_tile_kernel(const uint8_t* __restrict__ src, int32_t rows,
                                                       int32_t nblk, uint8_t* __restrict__ dst)
@@ -202,58 +273,26 @@ __global__ __launch_bounds__(256) void q4_tile_kernel(const uint8_t* __restrict_
     }
 }
 
-/* 16 fmas: S0 (vector b) and S1 (vector b+1) take terms 8p .. 8p+7 of the
- * block, in order, interleaved; x0..x3 hold the pair's values (lane n:
- * columns 4n..4n+3 of b, lane n+8: of b+1) and q0..q7 the weights. */
-#define G4S_FMAC_BCAST(N0, N1, N2, N3)                                                          \
-    asm("v_fmac_f32_dpp %0, %2, %6 row_newbcast:" N0 " row_mask:0xf bank_mask:0xf\n\t"          \
-        "v_fmac_f32_dpp %1, %2, %6 row_newbcast:" N1 " row_mask:0xf bank_mask:0xf\n\t"          \
-        "v_fmac_f32_dpp %0, %3, %7 row_newbcast:" N0 " row_mask:0xf bank_mask:0xf\n\t"          \
-        "v_fmac_f32_dpp %1, %3, %7 row_newbcast:" N1 " row_mask:0xf bank_mask:0xf\n\t"          \
-        "v_fmac_f32_dpp %0, %4, %8 row_newbcast:" N0 " row_mask:0xf bank_mask:0xf\n\t"          \
-        "v_fmac_f32_dpp %1, %4, %8 row_newbcast:" N1 " row_mask:0xf bank_mask:0xf\n\t"          \
-        "v_fmac_f32_dpp %0, %5, %9 row_newbcast:" N0 " row_mask:0xf bank_mask:0xf\n\t"          \
-        "v_fmac_f32_dpp %1, %5, %9 row_newbcast:" N1 " row_mask:0xf bank_mask:0xf\n\t"          \
-        "v_fmac_f32_dpp %0, %2, %10 row_newbcast:" N2 " row_mask:0xf bank_mask:0xf\n\t"         \
-        "v_fmac_f32_dpp %1, %2, %10 row_newbcast:" N3 " row_mask:0xf bank_mask:0xf\n\t"         \
-        "v_fmac_f32_dpp %0, %3, %11 row_newbcast:" N2 " row_mask:0xf bank_mask:0xf\n\t"         \
-        "v_fmac_f32_dpp %1, %3, %11 row_newbcast:" N3 " row_mask:0xf bank_mask:0xf\n\t"         \
-        "v_fmac_f32_dpp %0, %4, %12 row_newbcast:" N2 " row_mask:0xf bank_mask:0xf\n\t"         \
-        "v_fmac_f32_dpp %1, %4, %12 row_newbcast:" N3 " row_mask:0xf bank_mask:0xf\n\t"         \
-        "v_fmac_f32_dpp %0, %5, %13 row_newbcast:" N2 " row_mask:0xf bank_mask:0xf\n\t"         \
-        "v_fmac_f32_dpp %1, %5, %13 row_newbcast:" N3 " row_mask:0xf bank_mask:0xf"             \
-        : "+v"(S0), "+v"(S1)                                                                    \
-        : "v"(x0), "v"(x1), "v"(x2), "v"(x3), "v"(q0), "v"(q1), "v"(q2), "v"(q3), "v"(q4),      \
-          "v"(q5), "v"(q6), "v"(q7))
-
-/* The 64 terms of one block for vectors b and b+1 (x: the pair's values). */
-__device__ __forceinline__ void fma_pair(float& S0, float& S1, const float4 x, const float (&q)[32])
+/* The logit of row r = 64 g + lane for vector b: written where wanted, and
+ * the group's summary (its largest key, the lowest row holding it, and the
+ * largest key of the other rows). */
+__device__ __forceinline__ void put_logit(float v, int32_t b, int32_t r, int32_t rows, int lane,
+                                          int32_t g, int32_t ngroups, float* __restrict__ out,
+                                          int64_t stride, uint64_t* __restrict__ gsum)
 {
-    const float x0 = x.x, x1 = x.y, x2 = x.z, x3 = x.w;
-    {
-        const float q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
-        const float q4 = q[4], q5 = q[5], q6 = q[6], q7 = q[7];
-        G4S_FMAC_BCAST("0", "8", "1", "9");
-    }
-    {
-        const float q0 = q[8], q1 = q[9], q2 = q[10], q3 = q[11];
-        const float q4 = q[12], q5 = q[13], q6 = q[14], q7 = q[15];
-        G4S_FMAC_BCAST("2", "10", "3", "11");
-    }
-    {
-        const float q0 = q[16], q1 = q[17], q2 = q[18], q3 = q[19];
-        const float q4 = q[20], q5 = q[21], q6 = q[22], q7 = q[23];
-        G4S_FMAC_BCAST("4", "12", "5", "13");
-    }
-    {
-        const float q0 = q[24], q1 = q[25], q2 = q[26], q3 = q[27];
-        const float q4 = q[28], q5 = q[29], q6 = q[30], q7 = q[31];
-        G4S_FMAC_BCAST("6", "14", "7", "15");
+    const bool live = r < rows;
+    if (out && live) out[(int64_t)b * stride + r] = v;
+    if (gsum) {
+        const uint32_t key = live ? cand_key(v) : 0u;
+        const uint32_t kmax = wave_max_u32(key);
+        const uint32_t r6 = (uint32_t)__builtin_ctzll(__ballot(key == kmax));
+        const uint32_t k2 = wave_max_u32((uint32_t)lane == r6 ? 0u : key);
+        if (lane == 0) gsum[(int64_t)b * ngroups + g] = gsum_pack(kmax, r6, k2);
     }
 }
-#undef G4S_FMAC_BCAST
 
-__global__ __launch_bounds__(64 * kTileWaves) void lmhead_tiled_kernel(
+template <int NG, int DEPTH>
+__global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
     const uint8_t* __restrict__ tiles, int32_t rows, int32_t nblk, const float* __restrict__ h,
     int32_t cols, int32_t batch, float* __restrict__ out, int64_t stride, uint64_t* __restrict__ gsum,
     int32_t ngroups)
@@ -261,74 +300,152 @@ __global__ __launch_bounds__(64 * kTileWaves) void lmhead_tiled_kernel(
     const int lane = threadIdx.x & 63;
     const int32_t g = __builtin_amdgcn_readfirstlane(blockIdx.x * kTileWaves + (threadIdx.x >> 6));
     if (g >= ngroups) return; /* whole waves: no barrier below */
+    const int32_t b0 = blockIdx.y * (4 * NG);
     const int32_t r = g * kQ4TileRows + lane;
-    const float* tsc = reinterpret_cast<const float*>(tiles + (int64_t)g * nblk * kQ4TileBytes);
-    const uint4* tq = reinterpret_cast<const uint4*>(tiles + (int64_t)g * nblk * kQ4TileBytes +
-                                                     kQ4TileRows * 4);
-    const uint32_t ul = (uint32_t)lane;
-    constexpr int kTileF = kQ4TileBytes / 4;  /* floats per tile */
-    constexpr int kTileQ = kQ4TileBytes / 16; /* uint4 per tile */
-    /* lane's share of a pair load: vector 2p + (n >> 3), columns 4 (n & 7) .. +3 */
-    const int n = lane & 15;
-    const int32_t xlane = (n >> 3) * cols + 4 * (n & 7);
-    for (int32_t b0 = 0; b0 < batch; b0 += kTileB) {
-        /* offset of pair p's load: vectors past the batch read vector batch-1
-         * (any valid row; their sums are discarded) */
-        /* 32-bit byte offsets from the uniform base (the hidden matrix is
-         * below 2 GiB: checked by the launcher) */
-        const auto xload = [&](int p, int32_t k) -> float4 {
-            const int32_t ub = b0 + 2 * p;
-            const int32_t o = ub + 1 < batch ? ub * cols + xlane : (batch - 1) * cols + 4 * (n & 7);
-            const uint32_t byte = (uint32_t)(o + 32 * k) * 4u;
-            return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(h) + byte);
-        };
-        float S[kTileB];
+    const uint8_t* tp = tiles + (int64_t)g * nblk * kQ4TileBytes;
+    /* byte offsets of the lane's vectors (the hidden matrix is below 2 GiB:
+     * checked by the caller); vectors past the batch read vector batch - 1
+     * (any valid row; their sums are discarded) */
+    uint32_t xo[NG];
 #pragma unroll
-        for (int b = 0; b < kTileB; ++b) S[b] = 0.0f;
-        /* the first block's weights and vector pairs */
-        float sc = tsc[ul];
-        uint4 w = tq[ul];
-        float4 xr[kXAhead];
+    for (int i = 0; i < NG; ++i) {
+        const int32_t v = b0 + 4 * i + (lane & 3);
+        xo[i] = (uint32_t)((v < batch ? v : batch - 1) * cols + 2 * (lane >> 2)) * 4u;
+    }
+    float sc[DEPTH];
+    uint4 w[DEPTH];
+    float2 x[DEPTH][NG];
+    const auto fetch = [&](int d, int32_t k) {
+        const uint8_t* t = tp + (uint32_t)k * (uint32_t)kQ4TileBytes;
+        sc[d] = reinterpret_cast<const float*>(t)[lane];
+        w[d] = reinterpret_cast<const uint4*>(t + kQ4TileRows * 4)[lane];
+        const char* hk = reinterpret_cast<const char*>(h) + (uint32_t)k * 128u;
 #pragma unroll
-        for (int p = 0; p < kXAhead; ++p) xr[p] = xload(p, 0);
-        for (int32_t k = 0; k < nblk; ++k) {
-            float q[32];
-            q4_dequant32(w, sc, q);
-            const int32_t kn = k + 1 < nblk ? k + 1 : k;
-            sc = tsc[(uint32_t)(kn * kTileF) + ul];
-            w = tq[(uint32_t)(kn * kTileQ) + ul];
-            /* the scheduler keeps each load where it is issued: kXAhead pairs
-             * before its use, after the block's weight loads */
+        for (int i = 0; i < NG; ++i) x[d][i] = *reinterpret_cast<const float2*>(hk + xo[i]);
+    };
+    f32x4 S[NG];
+#pragma unroll
+    for (int i = 0; i < NG; ++i) S[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+        fetch(d, d < nblk ? d : nblk - 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    int32_t k = 0;
+    for (; k + DEPTH <= nblk; k += DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            mac32<NG>(S, w[d], sc[d], x[d]);
+            const int32_t kn = k + d + DEPTH;
+            fetch(d, kn < nblk ? kn : nblk - 1);
+            /* keeps each load where it is issued, DEPTH blocks before its use */
             __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int p = 0; p < kTileB / 2; ++p) {
-                const float4 x = xr[p % kXAhead];
-                /* the pair kXAhead ahead (wrapping into the next block) */
-                const int pa = p + kXAhead;
-                const int32_t ka = pa < kTileB / 2 ? k : kn;
-                xr[p % kXAhead] = xload(pa % (kTileB / 2), ka);
-                __builtin_amdgcn_sched_barrier(0);
-                fma_pair(S[2 * p], S[2 * p + 1], x, q);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        const bool live = r < rows;
-#pragma unroll
-        for (int b = 0; b < kTileB; ++b) {
-            if (b0 + b < batch) {
-                if (out && live) out[(int64_t)(b0 + b) * stride + r] = S[b];
-                if (gsum) {
-                    /* the group's summary: its largest key, the lowest row
-                     * holding it, and the largest key of the other rows */
-                    const uint32_t key = live ? cand_key(S[b]) : 0u;
-                    const uint32_t kmax = wave_max_u32(key);
-                    const uint32_t r6 = (uint32_t)__builtin_ctzll(__ballot(key == kmax));
-                    const uint32_t k2 = wave_max_u32(ul == r6 ? 0u : key);
-                    if (lane == 0) gsum[(int64_t)(b0 + b) * ngroups + g] = gsum_pack(kmax, r6, k2);
-                }
-            }
         }
     }
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+        if (k + d < nblk) mac32<NG>(S, w[d], sc[d], x[d]);
+#pragma unroll
+    for (int i = 0; i < 4 * NG; ++i)
+        if (b0 + i < batch)
+            put_logit(S[i / 4][i % 4], b0 + i, r, rows, lane, g, ngroups, out, stride, gsum);
+}
+
+/* Terms 8W .. 8W+7 of a block for one vector.  x: lane l holds columns
+ * 2 (l % 16) and 2 (l % 16) + 1; row_newbcast hands lane n's value to its
+ * 16-lane row, the same value in all four rows.  The s_nop covers the two
+ * wait states between a VALU write of x (a copy by the compiler) and its DPP
+ * read. */
+#define G4S_FMAC8(N0, N1, N2, N3)                                                               \
+    asm("s_nop 1\n\t"                                                                           \
+        "v_fmac_f32_dpp %0, %1, %3 row_newbcast:" N0 " row_mask:0xf bank_mask:0xf\n\t"          \
+        "v_fmac_f32_dpp %0, %2, %4 row_newbcast:" N0 " row_mask:0xf bank_mask:0xf\n\t"          \
+        "v_fmac_f32_dpp %0, %1, %5 row_newbcast:" N1 " row_mask:0xf bank_mask:0xf\n\t"          \
+        "v_fmac_f32_dpp %0, %2, %6 row_newbcast:" N1 " row_mask:0xf bank_mask:0xf\n\t"          \
+        "v_fmac_f32_dpp %0, %1, %7 row_newbcast:" N2 " row_mask:0xf bank_mask:0xf\n\t"          \
+        "v_fmac_f32_dpp %0, %2, %8 row_newbcast:" N2 " row_mask:0xf bank_mask:0xf\n\t"          \
+        "v_fmac_f32_dpp %0, %1, %9 row_newbcast:" N3 " row_mask:0xf bank_mask:0xf\n\t"          \
+        "v_fmac_f32_dpp %0, %2, %10 row_newbcast:" N3 " row_mask:0xf bank_mask:0xf"             \
+        : "+v"(S)                                                                               \
+        : "v"(x.x), "v"(x.y), "v"(q[0]), "v"(q[1]), "v"(q[2]), "v"(q[3]), "v"(q[4]), "v"(q[5]), \
+          "v"(q[6]), "v"(q[7]))
+template <int W>
+__device__ __forceinline__ void fmac8(float& S, const float (&q)[8], const float2 x)
+{
+    if constexpr (W == 0) G4S_FMAC8("0", "1", "2", "3");
+    if constexpr (W == 1) G4S_FMAC8("4", "5", "6", "7");
+    if constexpr (W == 2) G4S_FMAC8("8", "9", "10", "11");
+    if constexpr (W == 3) G4S_FMAC8("12", "13", "14", "15");
+}
+#undef G4S_FMAC8
+
+/* One or two hidden vectors per wave: one v_fmac_f32 with a DPP broadcast a
+ * term.  A matrix instruction would spend its four vectors' time on one. */
+template <int NV, int DEPTH>
+__global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_few_kernel(
+    const uint8_t* __restrict__ tiles, int32_t rows, int32_t nblk, const float* __restrict__ h,
+    int32_t cols, float* __restrict__ out, int64_t stride, uint64_t* __restrict__ gsum,
+    int32_t ngroups)
+{
+    const int lane = threadIdx.x & 63;
+    const int32_t g = __builtin_amdgcn_readfirstlane(blockIdx.x * kTileWaves + (threadIdx.x >> 6));
+    if (g >= ngroups) return; /* whole waves: no barrier below */
+    const int32_t b0 = blockIdx.y * NV;
+    const uint8_t* tp = tiles + (int64_t)g * nblk * kQ4TileBytes;
+    h += (int64_t)b0 * cols;
+    float sc[DEPTH];
+    uint4 w[DEPTH];
+    float2 x[DEPTH][NV];
+    const auto fetch = [&](int d, int32_t k) {
+        const uint8_t* t = tp + (uint32_t)k * (uint32_t)kQ4TileBytes;
+        sc[d] = reinterpret_cast<const float*>(t)[lane];
+        w[d] = reinterpret_cast<const uint4*>(t + kQ4TileRows * 4)[lane];
+#pragma unroll
+        for (int b = 0; b < NV; ++b)
+            x[d][b] = reinterpret_cast<const float2*>(h + (int64_t)b * cols + k * 32)[lane & 15];
+    };
+    float S[NV];
+#pragma unroll
+    for (int b = 0; b < NV; ++b) S[b] = 0.0f;
+    const auto term32 = [&](int d) {
+        const float s512 = 512.0f * sc[d], m8 = -8.0f * sc[d];
+        float q[8];
+        dequant8(w[d].x, s512, m8, q);
+#pragma unroll
+        for (int b = 0; b < NV; ++b) fmac8<0>(S[b], q, x[d][b]);
+        dequant8(w[d].y, s512, m8, q);
+#pragma unroll
+        for (int b = 0; b < NV; ++b) fmac8<1>(S[b], q, x[d][b]);
+        dequant8(w[d].z, s512, m8, q);
+#pragma unroll
+        for (int b = 0; b < NV; ++b) fmac8<2>(S[b], q, x[d][b]);
+        dequant8(w[d].w, s512, m8, q);
+#pragma unroll
+        for (int b = 0; b < NV; ++b) fmac8<3>(S[b], q, x[d][b]);
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+        fetch(d, d < nblk ? d : nblk - 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    int32_t k = 0;
+    for (; k + DEPTH <= nblk; k += DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            term32(d);
+            const int32_t kn = k + d + DEPTH;
+            fetch(d, kn < nblk ? kn : nblk - 1);
+            /* keeps each load where it is issued, DEPTH blocks before its use */
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+        if (k + d < nblk) term32(d);
+    const int32_t r = g * kQ4TileRows + lane;
+#pragma unroll
+    for (int b = 0; b < NV; ++b)
+        put_logit(S[b], b0 + b, r, rows, lane, g, ngroups, out, stride, gsum);
 }
 
 /* DoEmbeddingLookup for a Q4_0 table (src/Gemma4.Model.pas:2047-2080):
@@ -377,14 +494,55 @@ hipError_t q4_tile_launch(const uint8_t* src, int32_t rows, int32_t nblk, uint8_
     return hipGetLastError();
 }
 
+/* The split of a tiled launch into waves of 64 rows and some vectors:
+ *  - every (row group, vector) pair its own wave while that leaves at most
+ *    one wave per SIMD, and up to two vectors otherwise: the plain fma kernel
+ *    (2,560 columns: 20 us for 8,000 rows x 8 against 31 us with four vectors
+ *    a wave; 262,144 rows: 74 us for one vector against 105, 81 for two);
+ *  - else 4 * NG vectors a wave on the matrix cores, NG as large as needed
+ *    (up to 8) to leave at most one wave per SIMD (32,768 rows x 32: NG = 4
+ *    64 us, NG = 2 75, NG = 8 102; 262,144 rows x 32: NG = 8 366 us, NG = 4
+ *    416). */
+constexpr int32_t kLmSimds = 1024;
+
 hipError_t lmhead_tiled_launch(const uint8_t* tiles, int32_t rows, int32_t cols, const float* h,
                                int32_t batch, float* logits, int64_t stride, uint64_t* gsum,
                                hipStream_t s)
 {
     const int32_t ngroups = (rows + kQ4TileRows - 1) / kQ4TileRows;
-    const unsigned grid = (unsigned)((ngroups + kTileWaves - 1) / kTileWaves);
-    hipLaunchKernelGGL(lmhead_tiled_kernel, dim3(grid), dim3(64 * kTileWaves), 0, s, tiles, rows,
-                       cols / 32, h, cols, batch, logits, stride, gsum, ngroups);
+    const int32_t nblk = cols / 32;
+    const unsigned gx = (unsigned)((ngroups + kTileWaves - 1) / kTileWaves);
+    const dim3 block(64 * kTileWaves);
+    if (batch <= 2 || (int64_t)batch * ngroups <= kLmSimds) {
+        if ((int64_t)batch * ngroups <= kLmSimds || batch == 1)
+            hipLaunchKernelGGL((lmhead_tiled_few_kernel<1, 4>), dim3(gx, (unsigned)batch), block, 0,
+                               s, tiles, rows, nblk, h, cols, logits, stride, gsum, ngroups);
+        else
+            hipLaunchKernelGGL((lmhead_tiled_few_kernel<2, 4>), dim3(gx), block, 0, s, tiles, rows,
+                               nblk, h, cols, logits, stride, gsum, ngroups);
+        return hipGetLastError();
+    }
+    const int32_t quads = (batch + 3) / 4;
+    const int32_t fill = kLmSimds / ngroups;
+    int32_t passes = (quads + 7) / 8;
+    if (passes < fill) passes = fill < quads ? fill : quads;
+    const int32_t ng = (quads + passes - 1) / passes;
+    passes = (quads + ng - 1) / ng;
+    const dim3 grid(gx, (unsigned)passes);
+#define G4S_LM(NG, DEPTH)                                                                        \
+    hipLaunchKernelGGL((lmhead_tiled_kernel<NG, DEPTH>), grid, block, 0, s, tiles, rows, nblk, h,\
+                       cols, batch, logits, stride, gsum, ngroups)
+    switch (ng) {
+        case 1: G4S_LM(1, 4); break;
+        case 2: G4S_LM(2, 4); break;
+        case 3: G4S_LM(3, 3); break;
+        case 4: G4S_LM(4, 2); break;
+        case 5: G4S_LM(5, 2); break;
+        case 6: G4S_LM(6, 2); break;
+        case 7: G4S_LM(7, 2); break;
+        default: G4S_LM(8, 2); break;
+    }
+#undef G4S_LM
     return hipGetLastError();
 }
 

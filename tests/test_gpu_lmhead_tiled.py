@@ -119,6 +119,28 @@ def test_tiled_lmhead_bit_exact(orc, batch):
     s.close()
 
 
+@pytest.mark.parametrize("rows, cols, batches", [
+    # more row groups than SIMDs: two vectors a wave, then 4 * NG with NG = 1..8 and two passes
+    (64 * 1025 + 3, 96, [1, 2, 3, 4, 5, 9, 13, 17, 21, 25, 29, 32, 33]),
+    (64 * 1025, 32, [2, 3, 32]),       # one block per row
+    (64 * 513 + 1, 160, [2, 5, 8]),    # two vectors a wave, a partial last group
+    (64 * 100, 224, [10, 11, 48, 70]), # several slices of the batch
+    (64 * 11, 64, [93, 94, 200]),      # one vector a wave, then four
+])
+def test_tiled_lmhead_splits(orc, rows, cols, batches):
+    """Every split of rows and vectors over waves, with column blocks that the
+    prefetch depth does not divide and vectors that leave a wave partly empty."""
+    w = wl.host_q4_weights(rows + cols, rows, cols)
+    hidden = wl.host_hidden(rows, max(batches), cols)
+    want = orc.matvec_q4_batch(w, hidden, rows, cols, threads=8)
+    s = native.Sampler(V, max_batch=1, softcap=30.0)
+    for B in batches:
+        got = _tiled_lmhead(s, w, rows, cols, hidden[:B])
+        bad = got.view(np.uint32) != want[:B].view(np.uint32)
+        assert not bad.any(), f"B={B}: {bad.sum()} logits differ"
+    s.close()
+
+
 def test_tiled_lmhead_scale_edge_cases(orc):
     """Zero, subnormal (the engine's own widening), largest and negative fp16
     scales; tiny and large hidden values; one block per row."""
