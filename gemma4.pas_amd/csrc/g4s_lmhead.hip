@@ -176,6 +176,7 @@ __global__ __launch_bounds__(kLmBlock) void lmhead_q4_kernel(const uint8_t* __re
  * ------------------------------------------------------------------ */
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x32 __attribute__((ext_vector_type(32)));
 
 /* Eight weights of a row: nibble t of `w` is weight t.  A byte 0..15 read as
  * fp8 (e4m3) is n * 2^-9 (its denormals and first binade), so one
@@ -241,7 +242,7 @@ __device__ __forceinline__ void mac32(f32x4 (&S)[NG], const uint4 w, float sc, c
  * scale and 16 nibble bytes from the tile (256 + 1024 contiguous bytes per
  * wave) and two columns of its vectors (L1/L2 hits), kept DEPTH blocks ahead
  * in registers.  262,144 x 2,560 (a plain read of the 419 MB of tiles takes
- * 69-73 us): B = 1 645 -> 74 us, B = 8 138 us, B = 32 649 -> 366 us.
+ * 69-73 us): B = 1 645 -> 75 us, B = 8 152 us, B = 32 649 -> 361 us.
  * ------------------------------------------------------------------ */
 
 constexpr int kTileWaves = 4; /* waves (64-row groups) per workgroup */
@@ -349,6 +350,99 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
     for (int i = 0; i < 4 * NG; ++i)
         if (b0 + i < batch)
             put_logit(S[i / 4][i % 4], b0 + i, r, rows, lane, g, ngroups, out, stride, gsum);
+}
+
+/* Terms 8W .. 8W+7 of a block for 32 vectors.  x: lane l holds columns
+ * 8W + 4 (l / 32) .. + 3 of vector l % 32. */
+__device__ __forceinline__ void mac8x32(f32x32& S, const float (&q)[8], const float4 x)
+{
+    S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.x, q[0], S, 1, 0, 0);
+    S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.y, q[1], S, 1, 0, 0);
+    S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.z, q[2], S, 1, 0, 0);
+    S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.w, q[3], S, 1, 0, 0);
+    S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.x, q[4], S, 1, 1, 0);
+    S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.y, q[5], S, 1, 1, 0);
+    S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.z, q[6], S, 1, 1, 0);
+    S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.w, q[7], S, 1, 1, 0);
+}
+
+/* 32 vectors per wave on v_mfma_f32_32x32x1_2b: also one product per output,
+ * the weights' two blocks being rows 0-31 and 32-63 and CBSZ = 1 handing
+ * either half of the A register to both.  It reads eight times fewer operands
+ * per fma than the 4x4 form (262,144 x 2,560 x 32: 361 against 391 us). */
+template <int DEPTH>
+__global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled32_kernel(
+    const uint8_t* __restrict__ tiles, int32_t rows, int32_t nblk, const float* __restrict__ h,
+    int32_t cols, int32_t batch, float* __restrict__ out, int64_t stride, uint64_t* __restrict__ gsum,
+    int32_t ngroups)
+{
+    const int lane = threadIdx.x & 63;
+    const int32_t g = __builtin_amdgcn_readfirstlane(blockIdx.x * kTileWaves + (threadIdx.x >> 6));
+    if (g >= ngroups) return; /* whole waves: no barrier below */
+    const int32_t b0 = blockIdx.y * 32;
+    const uint8_t* tp = tiles + (int64_t)g * nblk * kQ4TileBytes;
+    /* vectors past the batch read vector batch - 1 (their sums are discarded) */
+    const int32_t v = b0 + (lane & 31);
+    const uint32_t xo = (uint32_t)((v < batch ? v : batch - 1) * cols + 4 * (lane >> 5)) * 4u;
+    float sc[DEPTH];
+    uint4 w[DEPTH];
+    float4 x[DEPTH][4];
+    const auto fetch = [&](int d, int32_t k) {
+        const uint8_t* t = tp + (uint32_t)k * (uint32_t)kQ4TileBytes;
+        sc[d] = reinterpret_cast<const float*>(t)[lane];
+        w[d] = reinterpret_cast<const uint4*>(t + kQ4TileRows * 4)[lane];
+        const char* hk = reinterpret_cast<const char*>(h) + (uint32_t)k * 128u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[d][i] = *reinterpret_cast<const float4*>(hk + xo + 32 * i);
+    };
+    f32x32 S;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) S[i] = 0.0f;
+    const auto term32 = [&](int d) {
+        const float s512 = 512.0f * sc[d], m8 = -8.0f * sc[d];
+        float q[8];
+        dequant8(w[d].x, s512, m8, q);
+        mac8x32(S, q, x[d][0]);
+        dequant8(w[d].y, s512, m8, q);
+        mac8x32(S, q, x[d][1]);
+        dequant8(w[d].z, s512, m8, q);
+        mac8x32(S, q, x[d][2]);
+        dequant8(w[d].w, s512, m8, q);
+        mac8x32(S, q, x[d][3]);
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+        fetch(d, d < nblk ? d : nblk - 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    int32_t k = 0;
+    for (; k + DEPTH <= nblk; k += DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            term32(d);
+            const int32_t kn = k + d + DEPTH;
+            fetch(d, kn < nblk ? kn : nblk - 1);
+            /* keeps each load where it is issued, DEPTH blocks before its use */
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+        if (k + d < nblk) term32(d);
+    const int32_t r = g * kQ4TileRows + lane;
+    /* register i: row lane % 32 (i < 16) or 32 + lane % 32 of vector
+     * 8 (i % 16 / 4) + 4 (lane / 32) + i % 4; swapping halves between i and
+     * i + 16 leaves lane = row, vectors c and c + 4 */
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(S[i]),
+                                                        __float_as_uint(S[i + 16]), false, false);
+        const int32_t c = b0 + 8 * (i / 4) + i % 4;
+        if (c < batch)
+            put_logit(__uint_as_float(y[0]), c, r, rows, lane, g, ngroups, out, stride, gsum);
+        if (c + 4 < batch)
+            put_logit(__uint_as_float(y[1]), c + 4, r, rows, lane, g, ngroups, out, stride, gsum);
+    }
 }
 
 /* Terms 8W .. 8W+7 of a block for one vector.  x: lane l holds columns
@@ -501,8 +595,8 @@ hipError_t q4_tile_launch(const uint8_t* src, int32_t rows, int32_t nblk, uint8_
  *    a wave; 262,144 rows: 74 us for one vector against 105, 81 for two);
  *  - else 4 * NG vectors a wave on the matrix cores, NG as large as needed
  *    (up to 8) to leave at most one wave per SIMD (32,768 rows x 32: NG = 4
- *    64 us, NG = 2 75, NG = 8 102; 262,144 rows x 32: NG = 8 366 us, NG = 4
- *    416). */
+ *    64 us, NG = 2 75, NG = 8 102; 262,144 rows x 32: NG = 8 391 us, NG = 4
+ *    416), and the 32-vector form where a wave takes 29 to 32. */
 constexpr int32_t kLmSimds = 1024;
 
 hipError_t lmhead_tiled_launch(const uint8_t* tiles, int32_t rows, int32_t cols, const float* h,
@@ -540,7 +634,10 @@ hipError_t lmhead_tiled_launch(const uint8_t* tiles, int32_t rows, int32_t cols,
         case 5: G4S_LM(5, 2); break;
         case 6: G4S_LM(6, 2); break;
         case 7: G4S_LM(7, 2); break;
-        default: G4S_LM(8, 2); break;
+        default:
+            hipLaunchKernelGGL(lmhead_tiled32_kernel<2>, grid, block, 0, s, tiles, rows, nblk, h,
+                               cols, batch, logits, stride, gsum, ngroups);
+            break;
     }
 #undef G4S_LM
     return hipGetLastError();
