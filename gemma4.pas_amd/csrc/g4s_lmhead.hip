@@ -16,22 +16,14 @@
  * least 2^-60 unless it is 0).  So the kernel is one fma per term, in the
  * reference's order.
  *
- * Layout: one weight row per thread (the TQ4Block row, 18 bytes per 32
- * weights, read in place), batch tiles of 32 hidden vectors whose values are
- * staged in LDS two blocks at a time (double-buffered, the next group's
- * loads in flight during the current one) and read as broadcasts; 32
- * independent running sums per thread.
- * Compute-bound at B=32: 2*B*rows*cols flops against 377 MB of weights.
+ * Every wave owns 64 weight rows (lane = row) and some hidden vectors: one
+ * accumulator form per number of vectors, over either layout of the weights.
  */
 #include "g4s_lmhead.h"
 
 namespace g4s {
 
 namespace {
-
-constexpr int kLmBlock = 256;
-constexpr int kLmTile = 32; /* hidden vectors per pass over the weights */
-constexpr int kLmKb = 2;    /* weight blocks (of 32 terms) per staged group of hidden values */
 
 /* TFloat16.ToSingle (src/Gemma4.Types.pas:438-481) as written, including its
  * handling of subnormal halves (the exponent is raised while normalising). */
@@ -58,100 +50,19 @@ __device__ __forceinline__ float f16_to_f32_ref(uint32_t v)
     return __uint_as_float(bits);
 }
 
-__global__ __launch_bounds__(kLmBlock) void lmhead_q4_kernel(const uint8_t* __restrict__ w,
-                                                             int32_t rows, int32_t nblk,
-                                                             const float* __restrict__ h,
-                                                             int32_t cols, int32_t batch,
-                                                             float* __restrict__ out,
-                                                             int64_t stride, int32_t h_vec4)
+/* The same value by the hardware's conversion: the two differ for subnormal
+ * halves only, whose exponent field the reference takes as 113 + shift where
+ * the value's is 113 - shift. */
+__device__ __forceinline__ float f16_to_f32_fast(uint32_t v)
 {
-    /* the hidden values of kLmKb weight blocks for the tile's kLmTile
-     * vectors, double-buffered: every lane reads the same entry (an LDS
-     * broadcast), so the fma operands come from VGPRs */
-    __shared__ __align__(16) float xs[2][kLmTile][kLmKb * 32];
-    constexpr int kStage = kLmTile * kLmKb * 8 / kLmBlock; /* float4 per thread per stage */
-    static_assert(kLmTile * kLmKb * 8 % kLmBlock == 0, "whole float4 stages");
-    const int32_t r = blockIdx.x * kLmBlock + threadIdx.x;
-    const bool active = r < rows;
-    const int32_t rr = active ? r : rows - 1;
-    const uint8_t* wrow = w + (int64_t)rr * nblk * 18;
-    const int32_t ngroup = (nblk + kLmKb - 1) / kLmKb;
-    for (int32_t b0 = 0; b0 < batch; b0 += kLmTile) {
-        const int32_t nb = batch - b0 < kLmTile ? batch - b0 : kLmTile;
-        /* hidden values of block group g (zeros past the batch or the row) */
-        const auto fetch = [&](int32_t g, float4 (&v)[kStage]) {
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) {
-                const int i = threadIdx.x + q * kLmBlock;
-                const int b = i / (kLmKb * 8), c4 = i % (kLmKb * 8);
-                const int32_t col = g * kLmKb * 32 + c4 * 4;
-                float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (b < nb && col < cols) {
-                    const float* src = h + (int64_t)(b0 + b) * cols + col;
-                    if (h_vec4)
-                        x = *reinterpret_cast<const float4*>(src);
-                    else
-                        x = make_float4(src[0], src[1], src[2], src[3]);
-                }
-                v[q] = x;
-            }
-        };
-        const auto stash = [&](int buf, const float4 (&v)[kStage]) {
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) {
-                const int i = threadIdx.x + q * kLmBlock;
-                reinterpret_cast<float4*>(&xs[buf][i / (kLmKb * 8)][0])[i % (kLmKb * 8)] = v[q];
-            }
-        };
-        float S[kLmTile];
-#pragma unroll
-        for (int b = 0; b < kLmTile; ++b) S[b] = 0.0f;
-        float4 nx[kStage];
-        fetch(0, nx);
-        stash(0, nx);
-        __syncthreads();
-        for (int32_t g = 0; g < ngroup; ++g) {
-            const int buf = g & 1;
-            if (g + 1 < ngroup) fetch(g + 1, nx); /* in flight during this group */
-            for (int kk = 0; kk < kLmKb; ++kk) {
-                const int32_t k = g * kLmKb + kk;
-                if (k >= nblk) break;
-                const uint16_t* blk = reinterpret_cast<const uint16_t*>(wrow + (int64_t)k * 18);
-                uint32_t half[9];
-#pragma unroll
-                for (int i = 0; i < 9; ++i) half[i] = blk[i];
-                const float sc = f16_to_f32_ref(half[0]);
-                float qs[32];
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const uint32_t byte = (half[1 + (j >> 1)] >> ((j & 1) * 8)) & 0xFFu;
-                    qs[2 * j] = (float)((int)(byte & 0x0Fu) - 8) * sc;     /* Tensors.pas:586 */
-                    qs[2 * j + 1] = (float)((int)(byte >> 4) - 8) * sc;    /* Tensors.pas:590 */
-                }
-                /* term j of every vector before term j+4: the 32 running sums
-                 * are independent chains, each still in the reference's order */
-#pragma unroll
-                for (int j4 = 0; j4 < 8; ++j4) {
-#pragma unroll
-                    for (int b = 0; b < kLmTile; ++b) {
-                        const float4 x = reinterpret_cast<const float4*>(&xs[buf][b][kk * 32])[j4];
-                        S[b] = __builtin_fmaf(qs[4 * j4], x.x, S[b]);
-                        S[b] = __builtin_fmaf(qs[4 * j4 + 1], x.y, S[b]);
-                        S[b] = __builtin_fmaf(qs[4 * j4 + 2], x.z, S[b]);
-                        S[b] = __builtin_fmaf(qs[4 * j4 + 3], x.w, S[b]);
-                    }
-                }
-            }
-            if (g + 1 < ngroup) stash(buf ^ 1, nx); /* read last in group g - 1 */
-            __syncthreads();
-        }
-        if (active) {
-#pragma unroll
-            for (int b = 0; b < kLmTile; ++b)
-                if (b < nb) out[(int64_t)(b0 + b) * stride + r] = S[b];
-        }
-        __syncthreads(); /* the next tile restages both buffers */
+    const _Float16 hv = __builtin_bit_cast(_Float16, (uint16_t)v);
+    float t = (float)hv;
+    const bool sub = __builtin_amdgcn_classh(hv, 0x90);
+    if (__ballot(sub)) {
+        const uint32_t u = __float_as_uint(t), e = (u >> 23) & 0xFFu;
+        if (sub) t = __uint_as_float(u + ((226u - 2u * e) << 23));
     }
+    return t;
 }
 
 /* ------------------------------------------------------------------
@@ -177,6 +88,10 @@ __global__ __launch_bounds__(kLmBlock) void lmhead_q4_kernel(const uint8_t* __re
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
+/* hidden values and row bytes may start on any element */
+typedef float float2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(1)));
 
 /* Eight weights of a row: nibble t of `w` is weight t.  A byte 0..15 read as
  * fp8 (e4m3) is n * 2^-9 (its denormals and first binade), so one
@@ -202,7 +117,7 @@ __device__ __forceinline__ void dequant8(uint32_t w, float s512, float m8, float
 /* Terms 8W .. 8W+7 of a block.  x[g]: lane l holds columns 2 (l / 4) and
  * 2 (l / 4) + 1 of vector 4g + l % 4. */
 template <int W, int NG>
-__device__ __forceinline__ void mac8(f32x4 (&S)[NG], const float (&q)[8], const float2 (&x)[NG])
+__device__ __forceinline__ void mac8(f32x4 (&S)[NG], const float (&q)[8], const float2u (&x)[NG])
 {
 #define G4S_MAC(T, C, AB)                                                                       \
     _Pragma("unroll") for (int g = 0; g < NG; ++g)                                              \
@@ -220,7 +135,7 @@ __device__ __forceinline__ void mac8(f32x4 (&S)[NG], const float (&q)[8], const 
 
 /* The 32 terms of one block. */
 template <int NG>
-__device__ __forceinline__ void mac32(f32x4 (&S)[NG], const uint4 w, float sc, const float2 (&x)[NG])
+__device__ __forceinline__ void mac32(f32x4 (&S)[NG], const uint4 w, float sc, const float2u (&x)[NG])
 {
     const float s512 = 512.0f * sc, m8 = -8.0f * sc;
     float q[8];
@@ -292,69 +207,51 @@ __device__ __forceinline__ void put_logit(float v, int32_t b, int32_t r, int32_t
     }
 }
 
-template <int NG, int DEPTH>
-__global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
-    const uint8_t* __restrict__ tiles, int32_t rows, int32_t nblk, const float* __restrict__ h,
-    int32_t cols, int32_t batch, float* __restrict__ out, int64_t stride, uint64_t* __restrict__ gsum,
-    int32_t ngroups)
-{
-    const int lane = threadIdx.x & 63;
-    const int32_t g = __builtin_amdgcn_readfirstlane(blockIdx.x * kTileWaves + (threadIdx.x >> 6));
-    if (g >= ngroups) return; /* whole waves: no barrier below */
-    const int32_t b0 = blockIdx.y * (4 * NG);
-    const int32_t r = g * kQ4TileRows + lane;
-    const uint8_t* tp = tiles + (int64_t)g * nblk * kQ4TileBytes;
-    /* byte offsets of the lane's vectors (the hidden matrix is below 2 GiB:
-     * checked by the caller); vectors past the batch read vector batch - 1
-     * (any valid row; their sums are discarded) */
-    uint32_t xo[NG];
-#pragma unroll
-    for (int i = 0; i < NG; ++i) {
-        const int32_t v = b0 + 4 * i + (lane & 3);
-        xo[i] = (uint32_t)((v < batch ? v : batch - 1) * cols + 2 * (lane >> 2)) * 4u;
-    }
-    float sc[DEPTH];
-    uint4 w[DEPTH];
-    float2 x[DEPTH][NG];
-    const auto fetch = [&](int d, int32_t k) {
-        const uint8_t* t = tp + (uint32_t)k * (uint32_t)kQ4TileBytes;
-        sc[d] = reinterpret_cast<const float*>(t)[lane];
-        w[d] = reinterpret_cast<const uint4*>(t + kQ4TileRows * 4)[lane];
-        const char* hk = reinterpret_cast<const char*>(h) + (uint32_t)k * 128u;
-#pragma unroll
-        for (int i = 0; i < NG; ++i) x[d][i] = *reinterpret_cast<const float2*>(hk + xo[i]);
+/* 4 * NG hidden vectors per wave.  Vectors past the batch read vector
+ * batch - 1 (any valid row; their sums are discarded).  Byte offsets stay
+ * within 32 bits: a launch's hidden matrix is below 2 GiB. */
+template <int NG>
+struct QuadAcc {
+    static constexpr int kVecs = 4 * NG;
+    struct X {
+        float2u v[NG];
     };
     f32x4 S[NG];
+    uint32_t xo[NG];
+    const char* hb;
+
+    __device__ __forceinline__ void init(const float* h, int32_t cols, int32_t b0, int32_t batch,
+                                         int lane)
+    {
+        hb = reinterpret_cast<const char*>(h);
 #pragma unroll
-    for (int i = 0; i < NG; ++i) S[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-        fetch(d, d < nblk ? d : nblk - 1);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    int32_t k = 0;
-    for (; k + DEPTH <= nblk; k += DEPTH) {
-#pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            mac32<NG>(S, w[d], sc[d], x[d]);
-            const int32_t kn = k + d + DEPTH;
-            fetch(d, kn < nblk ? kn : nblk - 1);
-            /* keeps each load where it is issued, DEPTH blocks before its use */
-            __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < NG; ++i) {
+            const int32_t v = b0 + 4 * i + (lane & 3);
+            xo[i] = (uint32_t)((v < batch ? v : batch - 1) * cols + 2 * (lane >> 2)) * 4u;
+            S[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
+    __device__ __forceinline__ void load(X& x, int32_t k) const
+    {
+        const char* hk = hb + (uint32_t)k * 128u;
 #pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d)
-        if (k + d < nblk) mac32<NG>(S, w[d], sc[d], x[d]);
+        for (int i = 0; i < NG; ++i) x.v[i] = *reinterpret_cast<const float2u*>(hk + xo[i]);
+    }
+    __device__ __forceinline__ void mac(const uint4 w, float sc, const X& x)
+    {
+        mac32<NG>(S, w, sc, x.v);
+    }
+    template <typename F>
+    __device__ __forceinline__ void emit(F put) const
+    {
 #pragma unroll
-    for (int i = 0; i < 4 * NG; ++i)
-        if (b0 + i < batch)
-            put_logit(S[i / 4][i % 4], b0 + i, r, rows, lane, g, ngroups, out, stride, gsum);
-}
+        for (int i = 0; i < 4 * NG; ++i) put(S[i / 4][i % 4], i);
+    }
+};
 
 /* Terms 8W .. 8W+7 of a block for 32 vectors.  x: lane l holds columns
  * 8W + 4 (l / 32) .. + 3 of vector l % 32. */
-__device__ __forceinline__ void mac8x32(f32x32& S, const float (&q)[8], const float4 x)
+__device__ __forceinline__ void mac8x32(f32x32& S, const float (&q)[8], const float4u x)
 {
     S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.x, q[0], S, 1, 0, 0);
     S = __builtin_amdgcn_mfma_f32_32x32x1f32(x.y, q[1], S, 1, 0, 0);
@@ -370,80 +267,59 @@ __device__ __forceinline__ void mac8x32(f32x32& S, const float (&q)[8], const fl
  * the weights' two blocks being rows 0-31 and 32-63 and CBSZ = 1 handing
  * either half of the A register to both.  It reads eight times fewer operands
  * per fma than the 4x4 form (262,144 x 2,560 x 32: 361 against 391 us). */
-template <int DEPTH>
-__global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled32_kernel(
-    const uint8_t* __restrict__ tiles, int32_t rows, int32_t nblk, const float* __restrict__ h,
-    int32_t cols, int32_t batch, float* __restrict__ out, int64_t stride, uint64_t* __restrict__ gsum,
-    int32_t ngroups)
-{
-    const int lane = threadIdx.x & 63;
-    const int32_t g = __builtin_amdgcn_readfirstlane(blockIdx.x * kTileWaves + (threadIdx.x >> 6));
-    if (g >= ngroups) return; /* whole waves: no barrier below */
-    const int32_t b0 = blockIdx.y * 32;
-    const uint8_t* tp = tiles + (int64_t)g * nblk * kQ4TileBytes;
-    /* vectors past the batch read vector batch - 1 (their sums are discarded) */
-    const int32_t v = b0 + (lane & 31);
-    const uint32_t xo = (uint32_t)((v < batch ? v : batch - 1) * cols + 4 * (lane >> 5)) * 4u;
-    float sc[DEPTH];
-    uint4 w[DEPTH];
-    float4 x[DEPTH][4];
-    const auto fetch = [&](int d, int32_t k) {
-        const uint8_t* t = tp + (uint32_t)k * (uint32_t)kQ4TileBytes;
-        sc[d] = reinterpret_cast<const float*>(t)[lane];
-        w[d] = reinterpret_cast<const uint4*>(t + kQ4TileRows * 4)[lane];
-        const char* hk = reinterpret_cast<const char*>(h) + (uint32_t)k * 128u;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[d][i] = *reinterpret_cast<const float4*>(hk + xo + 32 * i);
+struct WideAcc {
+    static constexpr int kVecs = 32;
+    struct X {
+        float4u v[4];
     };
     f32x32 S;
+    uint32_t xo;
+    const char* hb;
+
+    __device__ __forceinline__ void init(const float* h, int32_t cols, int32_t b0, int32_t batch,
+                                         int lane)
+    {
+        hb = reinterpret_cast<const char*>(h);
+        const int32_t v = b0 + (lane & 31);
+        xo = (uint32_t)((v < batch ? v : batch - 1) * cols + 4 * (lane >> 5)) * 4u;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) S[i] = 0.0f;
-    const auto term32 = [&](int d) {
-        const float s512 = 512.0f * sc[d], m8 = -8.0f * sc[d];
+        for (int i = 0; i < 32; ++i) S[i] = 0.0f;
+    }
+    __device__ __forceinline__ void load(X& x, int32_t k) const
+    {
+        const char* hk = hb + (uint32_t)k * 128u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x.v[i] = *reinterpret_cast<const float4u*>(hk + xo + 32 * i);
+    }
+    __device__ __forceinline__ void mac(const uint4 w, float sc, const X& x)
+    {
+        const float s512 = 512.0f * sc, m8 = -8.0f * sc;
         float q[8];
-        dequant8(w[d].x, s512, m8, q);
-        mac8x32(S, q, x[d][0]);
-        dequant8(w[d].y, s512, m8, q);
-        mac8x32(S, q, x[d][1]);
-        dequant8(w[d].z, s512, m8, q);
-        mac8x32(S, q, x[d][2]);
-        dequant8(w[d].w, s512, m8, q);
-        mac8x32(S, q, x[d][3]);
-    };
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-        fetch(d, d < nblk ? d : nblk - 1);
-        __builtin_amdgcn_sched_barrier(0);
+        dequant8(w.x, s512, m8, q);
+        mac8x32(S, q, x.v[0]);
+        dequant8(w.y, s512, m8, q);
+        mac8x32(S, q, x.v[1]);
+        dequant8(w.z, s512, m8, q);
+        mac8x32(S, q, x.v[2]);
+        dequant8(w.w, s512, m8, q);
+        mac8x32(S, q, x.v[3]);
     }
-    int32_t k = 0;
-    for (; k + DEPTH <= nblk; k += DEPTH) {
-#pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            term32(d);
-            const int32_t kn = k + d + DEPTH;
-            fetch(d, kn < nblk ? kn : nblk - 1);
-            /* keeps each load where it is issued, DEPTH blocks before its use */
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-#pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d)
-        if (k + d < nblk) term32(d);
-    const int32_t r = g * kQ4TileRows + lane;
     /* register i: row lane % 32 (i < 16) or 32 + lane % 32 of vector
      * 8 (i % 16 / 4) + 4 (lane / 32) + i % 4; swapping halves between i and
      * i + 16 leaves lane = row, vectors c and c + 4 */
+    template <typename F>
+    __device__ __forceinline__ void emit(F put) const
+    {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(S[i]),
-                                                        __float_as_uint(S[i + 16]), false, false);
-        const int32_t c = b0 + 8 * (i / 4) + i % 4;
-        if (c < batch)
-            put_logit(__uint_as_float(y[0]), c, r, rows, lane, g, ngroups, out, stride, gsum);
-        if (c + 4 < batch)
-            put_logit(__uint_as_float(y[1]), c + 4, r, rows, lane, g, ngroups, out, stride, gsum);
+        for (int i = 0; i < 16; ++i) {
+            const auto y = __builtin_amdgcn_permlane32_swap(
+                __float_as_uint(S[i]), __float_as_uint(S[i + 16]), false, false);
+            const int32_t c = 8 * (i / 4) + i % 4;
+            put(__uint_as_float(y[0]), c);
+            put(__uint_as_float(y[1]), c + 4);
+        }
     }
-}
+};
 
 /* Terms 8W .. 8W+7 of a block for one vector.  x: lane l holds columns
  * 2 (l % 16) and 2 (l % 16) + 1; row_newbcast hands lane n's value to its
@@ -464,7 +340,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled32_kernel(
         : "v"(x.x), "v"(x.y), "v"(q[0]), "v"(q[1]), "v"(q[2]), "v"(q[3]), "v"(q[4]), "v"(q[5]), \
           "v"(q[6]), "v"(q[7]))
 template <int W>
-__device__ __forceinline__ void fmac8(float& S, const float (&q)[8], const float2 x)
+__device__ __forceinline__ void fmac8(float& S, const float (&q)[8], const float2u x)
 {
     if constexpr (W == 0) G4S_FMAC8("0", "1", "2", "3");
     if constexpr (W == 1) G4S_FMAC8("4", "5", "6", "7");
@@ -475,47 +351,76 @@ __device__ __forceinline__ void fmac8(float& S, const float (&q)[8], const float
 
 /* One or two hidden vectors per wave: one v_fmac_f32 with a DPP broadcast a
  * term.  A matrix instruction would spend its four vectors' time on one. */
-template <int NV, int DEPTH>
-__global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_few_kernel(
+template <int NV>
+struct FewAcc {
+    static constexpr int kVecs = NV;
+    struct X {
+        float2u v[NV];
+    };
+    float S[NV];
+    const float* hb;
+    int32_t cols, at;
+
+    __device__ __forceinline__ void init(const float* h, int32_t c, int32_t b0, int32_t, int lane)
+    {
+        hb = h + (int64_t)b0 * c;
+        cols = c;
+        at = lane & 15;
+#pragma unroll
+        for (int b = 0; b < NV; ++b) S[b] = 0.0f;
+    }
+    __device__ __forceinline__ void load(X& x, int32_t k) const
+    {
+#pragma unroll
+        for (int b = 0; b < NV; ++b)
+            x.v[b] = reinterpret_cast<const float2u*>(hb + (int64_t)b * cols + k * 32)[at];
+    }
+    __device__ __forceinline__ void mac(const uint4 w, float sc, const X& x)
+    {
+        const float s512 = 512.0f * sc, m8 = -8.0f * sc;
+        float q[8];
+        dequant8(w.x, s512, m8, q);
+#pragma unroll
+        for (int b = 0; b < NV; ++b) fmac8<0>(S[b], q, x.v[b]);
+        dequant8(w.y, s512, m8, q);
+#pragma unroll
+        for (int b = 0; b < NV; ++b) fmac8<1>(S[b], q, x.v[b]);
+        dequant8(w.z, s512, m8, q);
+#pragma unroll
+        for (int b = 0; b < NV; ++b) fmac8<2>(S[b], q, x.v[b]);
+        dequant8(w.w, s512, m8, q);
+#pragma unroll
+        for (int b = 0; b < NV; ++b) fmac8<3>(S[b], q, x.v[b]);
+    }
+    template <typename F>
+    __device__ __forceinline__ void emit(F put) const
+    {
+#pragma unroll
+        for (int b = 0; b < NV; ++b) put(S[b], b);
+    }
+};
+
+template <typename Acc, int DEPTH>
+__global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
     const uint8_t* __restrict__ tiles, int32_t rows, int32_t nblk, const float* __restrict__ h,
-    int32_t cols, float* __restrict__ out, int64_t stride, uint64_t* __restrict__ gsum,
+    int32_t cols, int32_t batch, float* __restrict__ out, int64_t stride, uint64_t* __restrict__ gsum,
     int32_t ngroups)
 {
     const int lane = threadIdx.x & 63;
     const int32_t g = __builtin_amdgcn_readfirstlane(blockIdx.x * kTileWaves + (threadIdx.x >> 6));
     if (g >= ngroups) return; /* whole waves: no barrier below */
-    const int32_t b0 = blockIdx.y * NV;
+    const int32_t b0 = blockIdx.y * Acc::kVecs;
     const uint8_t* tp = tiles + (int64_t)g * nblk * kQ4TileBytes;
-    h += (int64_t)b0 * cols;
+    Acc acc;
+    acc.init(h, cols, b0, batch, lane);
     float sc[DEPTH];
     uint4 w[DEPTH];
-    float2 x[DEPTH][NV];
+    typename Acc::X x[DEPTH];
     const auto fetch = [&](int d, int32_t k) {
         const uint8_t* t = tp + (uint32_t)k * (uint32_t)kQ4TileBytes;
         sc[d] = reinterpret_cast<const float*>(t)[lane];
         w[d] = reinterpret_cast<const uint4*>(t + kQ4TileRows * 4)[lane];
-#pragma unroll
-        for (int b = 0; b < NV; ++b)
-            x[d][b] = reinterpret_cast<const float2*>(h + (int64_t)b * cols + k * 32)[lane & 15];
-    };
-    float S[NV];
-#pragma unroll
-    for (int b = 0; b < NV; ++b) S[b] = 0.0f;
-    const auto term32 = [&](int d) {
-        const float s512 = 512.0f * sc[d], m8 = -8.0f * sc[d];
-        float q[8];
-        dequant8(w[d].x, s512, m8, q);
-#pragma unroll
-        for (int b = 0; b < NV; ++b) fmac8<0>(S[b], q, x[d][b]);
-        dequant8(w[d].y, s512, m8, q);
-#pragma unroll
-        for (int b = 0; b < NV; ++b) fmac8<1>(S[b], q, x[d][b]);
-        dequant8(w[d].z, s512, m8, q);
-#pragma unroll
-        for (int b = 0; b < NV; ++b) fmac8<2>(S[b], q, x[d][b]);
-        dequant8(w[d].w, s512, m8, q);
-#pragma unroll
-        for (int b = 0; b < NV; ++b) fmac8<3>(S[b], q, x[d][b]);
+        acc.load(x[d], k);
     };
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
@@ -526,7 +431,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_few_kernel(
     for (; k + DEPTH <= nblk; k += DEPTH) {
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
-            term32(d);
+            acc.mac(w[d], sc[d], x[d]);
             const int32_t kn = k + d + DEPTH;
             fetch(d, kn < nblk ? kn : nblk - 1);
             /* keeps each load where it is issued, DEPTH blocks before its use */
@@ -535,11 +440,164 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_few_kernel(
     }
 #pragma unroll
     for (int d = 0; d < DEPTH - 1; ++d)
-        if (k + d < nblk) term32(d);
+        if (k + d < nblk) acc.mac(w[d], sc[d], x[d]);
     const int32_t r = g * kQ4TileRows + lane;
+    acc.emit([&](float v, int i) {
+        if (b0 + i < batch) put_logit(v, b0 + i, r, rows, lane, g, ngroups, out, stride, gsum);
+    });
+}
+
+/* ------------------------------------------------------------------
+ * The LM head on the engine's own rows (18-byte blocks).
+ *
+ * Read lane by lane, a wave's 64 rows are 64 cache lines per 18 bytes.  So a
+ * wave copies kRowKb blocks of its rows at a time into its own LDS (9 lanes
+ * read 144 bytes of a row, seven rows a load; held in registers while the
+ * previous stage is summed) and each lane then reads its own row from there.
+ * The LDS pitch is an odd number of dwords: no bank conflicts.  Three waves
+ * a SIMD (139 VGPRs with 32 vectors).
+ *
+ * 262,144 x 2,560: B = 1 652 -> 104 us, B = 8 692 -> 181, B = 32 750 -> 387
+ * (one row per thread before, 32 vectors' time for any batch).  B = 1 is
+ * bound by the weights' reads, which a stage's ends make 1.7 times their size
+ * (a line shared by two stages has left L2 in between: 12 waves a compute
+ * unit keep 50 MB in flight; without the sums 95 us).  16 blocks a stage at
+ * two waves a SIMD take 105, 187 and 387 us, and 100,003 x 1,120 for two
+ * vectors 36 us against 30; four waves a SIMD spill at 32 vectors (409 us).
+ * ------------------------------------------------------------------ */
+
+constexpr int kRowKb = 8;                                 /* blocks per stage */
+constexpr int kRowBytes = kRowKb * 18;
+constexpr int kRowChunks = kRowBytes / 16;                /* 16-byte loads per row and stage */
+constexpr int kRowPitch = kRowBytes / 4 + 1;              /* dwords */
+constexpr int kRowPer = 64 / kRowChunks;                  /* rows per load */
+constexpr int kRowLoads = (kQ4TileRows + kRowPer - 1) / kRowPer;
+constexpr int kRowEach = (kRowLoads + kRowKb / 2 - 1) / (kRowKb / 2); /* issued per block */
+static_assert(kRowBytes % 16 == 0, "whole 16-byte loads");
+
+/* 16 bytes at `a`, of which only those below `hi` are read (the others come back
+ * as anything); at least 16 bytes lie below `hi`. */
+__device__ __forceinline__ uint4 load16_within(const uint8_t* a, const uint8_t* hi)
+{
+    const uint8_t* at = a > hi - 16 ? hi - 16 : a;
+    const uint4u q = *reinterpret_cast<const uint4u*>(at);
+    const int64_t off = a - at; /* the wanted bytes are this much further up */
+    const int up = off > 15 ? 120 : (int)off * 8;
+    const uint64_t l = ((uint64_t)q.y << 32) | q.x, u = ((uint64_t)q.w << 32) | q.z;
+    const unsigned __int128 v = (((unsigned __int128)u << 64) | l) >> up;
+    const uint64_t vl = (uint64_t)v, vu = (uint64_t)(v >> 64);
+    return make_uint4((uint32_t)vl, (uint32_t)(vl >> 32), (uint32_t)vu, (uint32_t)(vu >> 32));
+}
+
+template <typename Acc, int DEPTH>
+__global__ __launch_bounds__(64, 3) void lmhead_rows_kernel(
+    const uint8_t* __restrict__ wt, int32_t rows, int32_t nblk, const float* __restrict__ h,
+    int32_t cols, int32_t batch, float* __restrict__ out, int64_t stride)
+{
+    static_assert(kRowKb % 2 == 0 && kRowKb % DEPTH == 0, "whole pairs, whole prefetch rounds");
+    __shared__ uint32_t stage[kQ4TileRows * kRowPitch];
+    const int lane = threadIdx.x;
+    const int32_t b0 = blockIdx.y * Acc::kVecs;
+    const int64_t pitch = (int64_t)nblk * 18;
+    const uint8_t* const wend = wt + (int64_t)rows * pitch;
+    const int32_t nstage = (nblk + kRowKb - 1) / kRowKb;
+    /* the last wave takes the last 64 rows and writes those that are its own */
+    const int32_t own = blockIdx.x * kQ4TileRows;
+    const int32_t r0 = own + kQ4TileRows <= rows ? own : rows > kQ4TileRows ? rows - kQ4TileRows : 0;
+    const uint8_t* const base = wt + (int64_t)r0 * pitch;
+    const int sub = lane / kRowChunks, chunk = lane % kRowChunks;
+    const uint32_t voff = (uint32_t)sub * (uint32_t)pitch + 16u * chunk;
+    /* lane's copies of load j: row kRowPer * j + sub */
+    const auto copies = [&](int j) { return sub < kRowPer && kRowPer * j + sub < kQ4TileRows; };
+    /* a stage whose copies could leave the weights: past the end of the last
+     * rows, or fewer than 64 rows at all */
+    const auto edge = [&](int32_t s) {
+        return base + (kQ4TileRows - 1) * pitch + (int64_t)(s + 1) * kRowBytes > wend;
+    };
+    uint4 st[kRowLoads];
+    const auto fetch = [&](int j, int32_t s) {
+        if (copies(j)) {
+            const uint4u q = *reinterpret_cast<const uint4u*>(
+                base + ((int64_t)s * kRowBytes + (int64_t)(kRowPer * j) * pitch) + voff);
+            st[j] = make_uint4(q.x, q.y, q.z, q.w);
+        }
+    };
+    uint32_t* const copy_to = stage + sub * kRowPitch + 4 * chunk;
+    const auto put = [&](int j, const uint4 v) {
+        if (copies(j)) {
+            uint32_t* d = copy_to + kRowPer * j * kRowPitch;
+            d[0] = v.x;
+            d[1] = v.y;
+            d[2] = v.z;
+            d[3] = v.w;
+        }
+    };
+    const uint32_t* const lrow = stage + lane * kRowPitch;
+    Acc acc;
+    acc.init(h, cols, b0, batch, lane);
+    typename Acc::X x[DEPTH];
+    if (!edge(0)) {
 #pragma unroll
-    for (int b = 0; b < NV; ++b)
-        put_logit(S[b], b0 + b, r, rows, lane, g, ngroups, out, stride, gsum);
+        for (int j = 0; j < kRowLoads; ++j) fetch(j, 0);
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) acc.load(x[d], d < nblk ? d : nblk - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int32_t s = 0; s < nstage; ++s) {
+        if (edge(s)) {
+#pragma unroll 6
+            for (int j = 0; j < kRowLoads; ++j)
+                put(j, load16_within(
+                           base + ((int64_t)s * kRowBytes + (int64_t)(kRowPer * j) * pitch) + voff,
+                           wend));
+        } else {
+#pragma unroll
+            for (int j = 0; j < kRowLoads; ++j) put(j, st[j]);
+        }
+        /* one wave: its LDS operations run in order */
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const bool more = s + 1 < nstage && !edge(s + 1);
+        uint32_t raw[2][9]; /* two blocks (36 bytes), read two blocks ahead */
+        const auto pair = [&](int p) {
+#pragma unroll
+            for (int i = 0; i < 9; ++i) raw[p & 1][i] = lrow[9 * p + i];
+        };
+        pair(0);
+#pragma unroll
+        for (int i = 0; i < kRowKb; ++i) {
+            const int32_t k = s * kRowKb + i;
+            if (k >= nblk) break;
+            if (more) {
+#pragma unroll
+                for (int j = kRowEach * i; j < kRowEach * (i + 1); ++j)
+                    if (j < kRowLoads) fetch(j, s + 1);
+            }
+            const uint32_t* e = raw[(i / 2) & 1];
+            uint32_t half;
+            uint4 w;
+            if (i % 2 == 0) {
+                if (i + 2 < kRowKb) pair(i / 2 + 1);
+                half = e[0] & 0xFFFFu;
+                w = make_uint4(
+                    __builtin_amdgcn_alignbit(e[1], e[0], 16), __builtin_amdgcn_alignbit(e[2], e[1], 16),
+                    __builtin_amdgcn_alignbit(e[3], e[2], 16), __builtin_amdgcn_alignbit(e[4], e[3], 16));
+            } else {
+                half = e[4] >> 16;
+                w = make_uint4(e[5], e[6], e[7], e[8]);
+            }
+            acc.mac(w, f16_to_f32_fast(half), x[i % DEPTH]);
+            const int32_t kn = k + DEPTH;
+            acc.load(x[i % DEPTH], kn < nblk ? kn : nblk - 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_wave_barrier(); /* the next stage is written after these reads */
+    }
+    const int32_t r = r0 + lane;
+    acc.emit([&](float v, int i) {
+        if (b0 + i < batch && r >= own && r < rows) out[(int64_t)(b0 + i) * stride + r] = v;
+    });
 }
 
 /* DoEmbeddingLookup for a Q4_0 table (src/Gemma4.Model.pas:2047-2080):
@@ -588,7 +646,7 @@ hipError_t q4_tile_launch(const uint8_t* src, int32_t rows, int32_t nblk, uint8_
     return hipGetLastError();
 }
 
-/* The split of a tiled launch into waves of 64 rows and some vectors:
+/* The split of a launch into waves of 64 rows and some vectors:
  *  - every (row group, vector) pair its own wave while that leaves at most
  *    one wave per SIMD, and up to two vectors otherwise: the plain fma kernel
  *    (2,560 columns: 20 us for 8,000 rows x 8 against 31 us with four vectors
@@ -596,8 +654,50 @@ hipError_t q4_tile_launch(const uint8_t* src, int32_t rows, int32_t nblk, uint8_
  *  - else 4 * NG vectors a wave on the matrix cores, NG as large as needed
  *    (up to 8) to leave at most one wave per SIMD (32,768 rows x 32: NG = 4
  *    64 us, NG = 2 75, NG = 8 102; 262,144 rows x 32: NG = 8 391 us, NG = 4
- *    416), and the 32-vector form where a wave takes 29 to 32. */
+ *    416), and the 32-vector form where a wave takes 29 to 32.
+ * launch(accumulator, prefetch depth, slices of the batch) starts the kernel. */
 constexpr int32_t kLmSimds = 1024;
+
+template <int D>
+struct Depth {
+    static constexpr int value = D;
+};
+
+template <typename F>
+void lmhead_split(int32_t ngroups, int32_t batch, F launch)
+{
+    if (batch <= 2 || (int64_t)batch * ngroups <= kLmSimds) {
+        if ((int64_t)batch * ngroups <= kLmSimds || batch == 1)
+            launch(FewAcc<1>{}, Depth<4>{}, batch);
+        else
+            launch(FewAcc<2>{}, Depth<4>{}, 1);
+        return;
+    }
+    const int32_t quads = (batch + 3) / 4;
+    const int32_t fill = kLmSimds / ngroups;
+    int32_t passes = (quads + 7) / 8;
+    if (passes < fill) passes = fill < quads ? fill : quads;
+    const int32_t ng = (quads + passes - 1) / passes;
+    passes = (quads + ng - 1) / ng;
+    switch (ng) {
+        case 1: launch(QuadAcc<1>{}, Depth<4>{}, passes); break;
+        case 2: launch(QuadAcc<2>{}, Depth<4>{}, passes); break;
+        case 3: launch(QuadAcc<3>{}, Depth<3>{}, passes); break;
+        case 4: launch(QuadAcc<4>{}, Depth<2>{}, passes); break;
+        case 5: launch(QuadAcc<5>{}, Depth<2>{}, passes); break;
+        case 6: launch(QuadAcc<6>{}, Depth<2>{}, passes); break;
+        case 7: launch(QuadAcc<7>{}, Depth<2>{}, passes); break;
+        default: launch(WideAcc{}, Depth<2>{}, passes); break;
+    }
+}
+
+/* Vectors of one launch: byte offsets into its hidden values stay within 31
+ * bits, its slices within a grid's second dimension. */
+int32_t lmhead_most(int32_t cols)
+{
+    const int64_t most = INT32_MAX / ((int64_t)cols * 4);
+    return (int32_t)(most < 1 ? 1 : most > 65535 ? 65535 : most);
+}
 
 hipError_t lmhead_tiled_launch(const uint8_t* tiles, int32_t rows, int32_t cols, const float* h,
                                int32_t batch, float* logits, int64_t stride, uint64_t* gsum,
@@ -606,51 +706,44 @@ hipError_t lmhead_tiled_launch(const uint8_t* tiles, int32_t rows, int32_t cols,
     const int32_t ngroups = (rows + kQ4TileRows - 1) / kQ4TileRows;
     const int32_t nblk = cols / 32;
     const unsigned gx = (unsigned)((ngroups + kTileWaves - 1) / kTileWaves);
-    const dim3 block(64 * kTileWaves);
-    if (batch <= 2 || (int64_t)batch * ngroups <= kLmSimds) {
-        if ((int64_t)batch * ngroups <= kLmSimds || batch == 1)
-            hipLaunchKernelGGL((lmhead_tiled_few_kernel<1, 4>), dim3(gx, (unsigned)batch), block, 0,
-                               s, tiles, rows, nblk, h, cols, logits, stride, gsum, ngroups);
-        else
-            hipLaunchKernelGGL((lmhead_tiled_few_kernel<2, 4>), dim3(gx), block, 0, s, tiles, rows,
-                               nblk, h, cols, logits, stride, gsum, ngroups);
-        return hipGetLastError();
+    const int32_t most = lmhead_most(cols);
+    for (int32_t b0 = 0; b0 < batch; b0 += most) {
+        const int32_t n = batch - b0 < most ? batch - b0 : most;
+        const float* hb = h + (int64_t)b0 * cols;
+        float* lb = logits ? logits + (int64_t)b0 * stride : nullptr;
+        uint64_t* gb = gsum ? gsum + (int64_t)b0 * ngroups : nullptr;
+        lmhead_split(ngroups, n, [&](auto acc, auto depth, int32_t passes) {
+            hipLaunchKernelGGL((lmhead_tiled_kernel<decltype(acc), decltype(depth)::value>),
+                               dim3(gx, (unsigned)passes), dim3(64 * kTileWaves), 0, s, tiles, rows,
+                               nblk, hb, cols, n, lb, stride, gb, ngroups);
+        });
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
     }
-    const int32_t quads = (batch + 3) / 4;
-    const int32_t fill = kLmSimds / ngroups;
-    int32_t passes = (quads + 7) / 8;
-    if (passes < fill) passes = fill < quads ? fill : quads;
-    const int32_t ng = (quads + passes - 1) / passes;
-    passes = (quads + ng - 1) / ng;
-    const dim3 grid(gx, (unsigned)passes);
-#define G4S_LM(NG, DEPTH)                                                                        \
-    hipLaunchKernelGGL((lmhead_tiled_kernel<NG, DEPTH>), grid, block, 0, s, tiles, rows, nblk, h,\
-                       cols, batch, logits, stride, gsum, ngroups)
-    switch (ng) {
-        case 1: G4S_LM(1, 4); break;
-        case 2: G4S_LM(2, 4); break;
-        case 3: G4S_LM(3, 3); break;
-        case 4: G4S_LM(4, 2); break;
-        case 5: G4S_LM(5, 2); break;
-        case 6: G4S_LM(6, 2); break;
-        case 7: G4S_LM(7, 2); break;
-        default:
-            hipLaunchKernelGGL(lmhead_tiled32_kernel<2>, grid, block, 0, s, tiles, rows, nblk, h,
-                               cols, batch, logits, stride, gsum, ngroups);
-            break;
-    }
-#undef G4S_LM
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 hipError_t lmhead_q4_0_launch(const uint8_t* w, int32_t rows, int32_t cols, const float* h,
                               int32_t batch, float* logits, int64_t stride, hipStream_t s)
 {
+    const int32_t ngroups = (rows + kQ4TileRows - 1) / kQ4TileRows;
     const int32_t nblk = cols / 32;
-    const int32_t h_vec4 = (reinterpret_cast<uintptr_t>(h) & 15u) == 0 ? 1 : 0;
-    hipLaunchKernelGGL(lmhead_q4_kernel, dim3((unsigned)((rows + kLmBlock - 1) / kLmBlock)),
-                       dim3(kLmBlock), 0, s, w, rows, nblk, h, cols, batch, logits, stride, h_vec4);
-    return hipGetLastError();
+    const int32_t most = lmhead_most(cols);
+    for (int32_t b0 = 0; b0 < batch; b0 += most) {
+        const int32_t n = batch - b0 < most ? batch - b0 : most;
+        const float* hb = h + (int64_t)b0 * cols;
+        float* lb = logits + (int64_t)b0 * stride;
+        lmhead_split(ngroups, n, [&](auto acc, auto depth, int32_t passes) {
+            /* prefetch distance in a stage of kRowKb blocks: a power of two */
+            constexpr int D = decltype(depth)::value == 3 ? 4 : decltype(depth)::value;
+            const dim3 grid((unsigned)ngroups, (unsigned)passes);
+            hipLaunchKernelGGL((lmhead_rows_kernel<decltype(acc), D>), grid, dim3(64), 0, s, w, rows,
+                               nblk, hb, cols, n, lb, stride);
+        });
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace g4s

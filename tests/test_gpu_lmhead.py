@@ -45,10 +45,8 @@ def test_lmhead_small_bit_exact(orc, batch):
 
 
 def test_lmhead_odd_block_count_and_unaligned_hidden(orc):
-    """An odd number of Q4_0 blocks per row (the kernel stages hidden values
-    two blocks at a time, so the last group is half empty) and a hidden
-    matrix that starts 4 bytes past a 16-byte boundary (staged with scalar
-    loads instead of 16-byte ones)."""
+    """An odd number of Q4_0 blocks per row and a hidden matrix that starts 4
+    bytes past a 16-byte boundary."""
     rows, cols, B = 300, 5 * 32, 3
     w = wl.host_q4_weights(81, rows, cols)
     hidden = wl.host_hidden(82, B, cols)
@@ -63,6 +61,42 @@ def test_lmhead_odd_block_count_and_unaligned_hidden(orc):
     want = orc.matvec_q4_batch(w, hidden, rows, cols)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), \
         f"{np.sum(got != want)} logits differ"
+    s.close()
+
+
+@pytest.mark.parametrize("rows, cols, batches", [
+    (1, 32, [1, 5]), (63, 16 * 32, [1, 33]),               # fewer rows than a wave has
+    (64, 15 * 32, [1, 2]), (65, 17 * 32, [1, 3]),          # a partial and a second stage of blocks
+    (127, 33 * 32, [1, 9]), (64 * 3 + 1, 32, [7]),         # odd row pitch; rows shorter than a stage
+    (64 * 100, 7 * 32, [10, 11, 48, 70]),                  # several slices of the batch
+    # more row groups than SIMDs: two vectors a wave, then 4 * NG with NG = 1..8 and two passes
+    (64 * 1025 + 3, 3 * 32, [1, 2, 3, 5, 9, 13, 17, 21, 25, 32, 33]),
+    (64 * 1025, 18 * 32, [1, 2, 8, 32]),
+])
+@pytest.mark.parametrize("shift", [0, 2, 5])
+def test_lmhead_rows_splits(orc, rows, cols, batches, shift):
+    """Every split of rows and vectors over waves, stages that the block count
+    does not fill, rows that start on any byte, and weights that fill their
+    buffer to the last byte."""
+    if shift == 5 and rows > 1000:
+        pytest.skip("the same kernels as shift 2")
+    w = wl.host_q4_weights(rows + cols, rows, cols)
+    hidden = wl.host_hidden(rows, max(batches), cols)
+    want = orc.matvec_q4_batch(w, hidden, rows, cols, threads=8)
+    s = native.Sampler(V, max_batch=1, softcap=30.0)
+    dw = hip.Buffer(w.nbytes + shift)
+    dw.upload(w, offset=shift)
+    dh = hip.Buffer(4 * (hidden.size + 1))
+    dh.upload(np.ascontiguousarray(hidden, F32), offset=4)
+    stride = rows + 1
+    for B in batches:
+        dl = hip.Buffer.from_array(np.full((B, stride), 7.0, F32))
+        s.lmhead_q4_0(dw.offset(shift), rows, cols, dh.offset(4), B, dl, stride)
+        hip.synchronize()
+        got = dl.download(F32).reshape(B, stride)
+        bad = got[:, :rows].view(np.uint32) != want[:B].view(np.uint32)
+        assert not bad.any(), f"B={B}: {bad.sum()} logits differ"
+        assert np.all(got[:, rows] == 7.0)
     s.close()
 
 
