@@ -92,37 +92,29 @@ __device__ __forceinline__ uint32_t ent_idx(uint64_t e) { return (uint32_t)e; }
 
 /* Four consecutive elements from e0 (a multiple of 4); elements at or beyond
  * `limit` are -inf (never screened into the heap: -inf <= -1e30). */
-template <int DT>
 __device__ __forceinline__ void load4(const char* row, int64_t e0, int64_t limit, float (&v)[4])
 {
     if (e0 + 4 <= limit) {
-        if constexpr (DT == 0) {
-            const float4 q = *reinterpret_cast<const float4*>(row + e0 * 4);
-            v[0] = q.x;
-            v[1] = q.y;
-            v[2] = q.z;
-            v[3] = q.w;
-        } else {
-            const uint2 q = *reinterpret_cast<const uint2*>(row + e0 * 2);
-            v[0] = __uint_as_float(q.x << 16);
-            v[1] = __uint_as_float(q.x & 0xFFFF0000u);
-            v[2] = __uint_as_float(q.y << 16);
-            v[3] = __uint_as_float(q.y & 0xFFFF0000u);
-        }
+        const float4 q = *reinterpret_cast<const float4*>(row + e0 * 4);
+        v[0] = q.x;
+        v[1] = q.y;
+        v[2] = q.z;
+        v[3] = q.w;
     } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            v[i] = (e0 + i < limit) ? load_elem<DT>(row, e0 + i) : -__builtin_inff();
+            v[i] = (e0 + i < limit) ? load_elem<0>(row, e0 + i) : -__builtin_inff();
     }
 }
 
-/* The reference's min-heap pass (Model.pas:2632-2664) over the whole row:
+/* The reference's min-heap pass (Model.pas:2632-2664) over a whole binary32
+ * row (bf16 rows, where ties are ordinary: topk_replay_kernel):
  * tiles of 1024 elements screened against the current root (an element at
  * or below it would be rejected by every later root too), the screened ones
  * inserted in index order by one lane with the reference's comparisons; the
  * next tile is loaded while one is screened.  On return hv[0..K) / hi[0..K)
  * hold the heap (hi = -1 where the row had fewer than K logits above -1e30). */
-template <int DT, typename SH>
+template <typename SH>
 __device__ void replay_heap(const char* row, int V, int K, SH& sh, float* hv, int32_t* hi)
 {
     float* qv = reinterpret_cast<float*>(sh.mc);
@@ -134,10 +126,10 @@ __device__ void replay_heap(const char* row, int V, int K, SH& sh, float* hv, in
     }
     __syncthreads();
     float cur[4];
-    load4<DT>(row, (int64_t)tid * 4, V, cur);
+    load4(row, (int64_t)tid * 4, V, cur);
     for (int base = 0; base < V; base += kDTile) {
         float nxt[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (base + kDTile < V) load4<DT>(row, (int64_t)base + kDTile + (int64_t)tid * 4, V, nxt);
+        if (base + kDTile < V) load4(row, (int64_t)base + kDTile + (int64_t)tid * 4, V, nxt);
         const float root = hv[0];
         int take = 0;
 #pragma unroll
@@ -367,6 +359,8 @@ __global__ __launch_bounds__(kDB) void topk_decode_kernel(TopkArgs a)
 
     /* ------------------------------------------------------------ merge */
     uint32_t flags = G4S_FLAG_TOPK_PATH;
+    if constexpr (DT == 1)
+        if (tid == 0) st_dev(&a.wbounds[(int64_t)row * kWaveBounds], 0u); /* no replay */
     /* thread t: the lists of workgroup t (its four waves), one round trip of
      * device-coherent 16-byte loads */
     constexpr int kE = kDW * kDL;
@@ -723,9 +717,13 @@ __global__ __launch_bounds__(kDB) void topk_decode_kernel(TopkArgs a)
 
         if (mode == 2) {
             flags |= G4S_FLAG_HEAP_REPLAY;
+            if constexpr (DT == 1) { /* topk_replay_kernel takes the row */
+                if (tid == 0) st_dev(&a.wbounds[(int64_t)row * kWaveBounds], flags);
+                return;
+            }
             float* hv = reinterpret_cast<float*>(sh.surv);
             int32_t* hi = reinterpret_cast<int32_t*>(sh.surv) + KMAX;
-            replay_heap<DT>(rowp, V, K, sh, hv, hi);
+            replay_heap(rowp, V, K, sh, hv, hi);
             /* keep the entries holding an index (Model.pas:2668-2676), then
              * rank them by index (:2678-2688) */
             if (tid < K) sh.ix[tid] = hi[tid] >= 0 ? (uint32_t)hi[tid] : 0xFFFFFFFFu;

@@ -149,8 +149,8 @@ struct FullWorkspace {
     uint32_t* hist = nullptr;    /* [max_batch][kWideBins], zero between launches */
     TieRec* ties = nullptr;      /* [max_batch][kSelMaxChunks] */
     uint32_t* bits = nullptr;    /* [max_batch][ceil(vocab/32)] surviving tied copies */
-    float* heap_v = nullptr;     /* [vocab] replay heap (one row at a time) */
-    int32_t* heap_i = nullptr;   /* [vocab] */
+    uint64_t* heap = nullptr;    /* [vocab + kHeapExtra] replay heap of rows that LDS does not
+                                    hold (one row at a time) */
     /* streaming pipeline of full bf16 rows */
     float* ytab = nullptr;       /* [65536] y = softcap(x) of every bf16 code (full-row form) */
     FbRow* fbrow = nullptr;      /* [max_batch] */

@@ -59,6 +59,7 @@
 #include <climits>
 
 #include "g4s_fullcore.h"
+#include "g4s_heap.h"
 
 namespace g4s {
 
@@ -304,76 +305,52 @@ __global__ __launch_bounds__(kFullBlock) void wide_ties_find_kernel(FullArgs a)
     }
 }
 
-/* Exact replay of the reference's min-heap pass (Model.pas:2632-2664) for
- * the rows whose tie at tau depends on the heap layout, one row at a time
- * with the heap in device memory.  One wave screens 64 logits per step
- * against the current root; lane 0 inserts the ones that pass, in index
- * order.  The surviving copies of tau are then marked in the row's bitmask.
- * Cost: about (K + K ln(V/K)) log2(K) dependent heap steps per row. */
+/* Exact replay of the reference's min-heap pass (Model.pas:2632-2664,
+ * g4s_heap.h) for the rows whose tie at tau depends on the heap layout; the
+ * surviving copies of tau are then marked in the row's bitmask.  One
+ * workgroup per row with the heap in LDS; the rows whose K does not fit
+ * there share one heap in device memory, one after another. */
+constexpr int kWrBlock = 512;
+constexpr int kWrHeap = 16384 - 1024; /* LDS heap entries (120 KiB) */
+constexpr int kWrQueue = 2048;
+
 template <int DT>
-__global__ __launch_bounds__(64) void wide_replay_kernel(FullArgs a)
+__global__ __launch_bounds__(kWrBlock) void wide_replay_kernel(FullArgs a)
 {
-    const int lane = threadIdx.x;
+    __shared__ alignas(16) uint64_t lheap[kWrHeap];
+    __shared__ uint64_t q[kWrQueue];
+    __shared__ HeapCtl ctl;
+    const int tid = threadIdx.x;
     const int V = a.vocab;
-    float* hv = a.ws.heap_v;
-    int32_t* hi = a.ws.heap_i;
-    for (int row = 0; row < a.batch; ++row) {
+    const auto replay = [&](int row, bool big) {
         const RowIn ri = row_in(a, row);
-        if (row_class(a, ri.p.top_k) != kRowWide) continue;
+        if (row_class(a, ri.p.top_k) != kRowWide) return;
         WideSel* sp = a.ws.sel + row;
         const WideSel s = *sp;
-        if (s.state != kSelReplay) continue;
         const int K = ri.p.top_k;
+        if (s.state != kSelReplay || (K + kHeapExtra > kWrHeap) != big) return;
         const char* rowp = row_ptr<DT>(a, row);
-        if (lane == 0) {
-            for (int i = 0; i < K; ++i) { /* :2634-2638 */
-                hv[i] = -1e30f;
-                hi[i] = -1;
-            }
+        uint64_t* heap = lheap;
+        if (big) {
+            heap = a.ws.heap;
+            heap_replay<kWrBlock, DT>(rowp, V, K, heap, q, kWrQueue, ctl);
+        } else {
+            heap_replay<kWrBlock, DT>(rowp, V, K, lheap, q, kWrQueue, ctl);
         }
-        float root = -1e30f;
-        for (int base = 0; base < V; base += 64) {
-            const int e = base + lane;
-            float x = 0.0f;
-            if (e < V) {
-                if constexpr (DT == 0)
-                    x = reinterpret_cast<const float*>(rowp)[e];
-                else
-                    x = __uint_as_float((uint32_t)reinterpret_cast<const uint16_t*>(rowp)[e] << 16);
-            }
-            uint64_t take = __ballot(e < V && !(x <= root));
-            while (take) {
-                const int l = (int)__builtin_ctzll(take);
-                take &= take - 1;
-                const float v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
-                if (lane == 0 && !(v <= hv[0])) { /* :2643-2644 */
-                    int p = 0;
-                    for (;;) { /* :2647-2661 */
-                        int c = p * 2 + 1;
-                        if (c >= K) break;
-                        if (c + 1 < K && hv[c + 1] < hv[c]) c += 1;
-                        if (hv[c] >= v) break;
-                        hv[p] = hv[c];
-                        hi[p] = hi[c];
-                        p = c;
-                    }
-                    hv[p] = v;
-                    hi[p] = base + l;
-                }
-            }
-            const float r0 = lane == 0 ? hv[0] : 0.0f;
-            root = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r0), 0));
+        uint32_t* bits = a.ws.bits + (int64_t)row * a.ws.bits_stride;
+        for (int w = tid; w < a.ws.bits_stride; w += kWrBlock) bits[w] = 0u;
+        __syncthreads();
+        for (int i = 1 + tid; i <= K; i += kWrBlock) {
+            const int32_t idx = heap_idx(heap[i]);
+            if (idx >= 0 && cand_key(heap_val(heap[i])) == s.tau)
+                atomicOr(&bits[idx >> 5], 1u << (idx & 31));
         }
-        if (lane == 0) {
-            uint32_t* bits = a.ws.bits + (int64_t)row * a.ws.bits_stride;
-            for (int w = 0; w < a.ws.bits_stride; ++w) bits[w] = 0u;
-            for (int i = 0; i < K; ++i) {
-                const int32_t idx = hi[i];
-                if (idx >= 0 && cand_key(hv[i]) == s.tau) bits[idx >> 5] |= 1u << (idx & 31);
-            }
-            sp->state = kSelBits;
-        }
-    }
+        __syncthreads();
+        if (tid == 0) sp->state = kSelBits;
+    };
+    replay(blockIdx.x, false);
+    if (blockIdx.x == 0)
+        for (int row = 0; row < a.batch; ++row) replay(row, true);
 }
 
 /* ------------------------------------------------------------ 1: max */
@@ -1003,8 +980,8 @@ hipError_t full_alloc(FullWorkspace& ws, int32_t vocab, int32_t max_batch)
     if (e == hipSuccess) e = hipMalloc((void**)&ws.ties, mb * kSelMaxChunks * sizeof(TieRec));
     if (e == hipSuccess)
         e = hipMalloc((void**)&ws.bits, mb * (size_t)ws.bits_stride * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.heap_v, (size_t)vocab * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.heap_i, (size_t)vocab * sizeof(int32_t));
+    if (e == hipSuccess)
+        e = hipMalloc((void**)&ws.heap, ((size_t)vocab + kHeapExtra) * sizeof(uint64_t));
     if (e == hipSuccess) e = hipMalloc((void**)&ws.ytab, (size_t)65536 * sizeof(float));
     if (e == hipSuccess) e = hipMalloc((void**)&ws.fbrow, mb * sizeof(FbRow));
     if (e == hipSuccess) e = hipMalloc((void**)&ws.etab8, mb * kBfTab * sizeof(float));
@@ -1018,7 +995,7 @@ hipError_t full_alloc(FullWorkspace& ws, int32_t vocab, int32_t max_batch)
 void full_free(FullWorkspace& ws)
 {
     void* ptrs[] = {ws.rows, ws.chunks, ws.lmap, ws.cmap, ws.beta_l, ws.beta_c, ws.etab, ws.ptab, ws.tmask,
-                    ws.sel, ws.hist, ws.ties, ws.bits, ws.heap_v, ws.heap_i, ws.ytab, ws.fbrow,
+                    ws.sel, ws.hist, ws.ties, ws.bits, ws.heap, ws.ytab, ws.fbrow,
                     ws.etab8, ws.ptab8, ws.stage, ws.cpost, ws.head};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -1111,7 +1088,8 @@ static hipError_t launch_dt(const FullArgs& a0, hipStream_t s)
         }
         hipLaunchKernelGGL((wide_ties_kernel<DT>), sel, dim3(kFullBlock), 0, s, a);
         hipLaunchKernelGGL((wide_ties_find_kernel<DT>), rows, dim3(kFullBlock), 0, s, a);
-        hipLaunchKernelGGL((wide_replay_kernel<DT>), dim3(1), dim3(64), 0, s, a);
+        hipLaunchKernelGGL((wide_replay_kernel<DT>), dim3((unsigned)a.batch), dim3(kWrBlock), 0, s,
+                           a);
     }
     hipLaunchKernelGGL((full_max_kernel<DT>), waves, dim3(kFullBlock), 0, s, a);
     hipLaunchKernelGGL((full_row_kernel<DT>),

@@ -41,6 +41,7 @@
  *      sum against fl32(u*TopP).  The sequential sums are exact left-to-right
  *      binary32 chains over broadcast LDS reads.
  */
+#include "g4s_heap.h"
 #include "g4s_select.h"
 #include "g4s_topk.h"
 #include "g4s_lmhead.h"
@@ -88,12 +89,12 @@ struct TopkShared {
 /* ------------------------------------------------------------ heap replay */
 
 /* Exact replay of the reference's min-heap pass (Model.pas:2632-2664) over a
- * whole row, for rows whose K-th value is tied in a way the heap layout
- * decides.  Elements are screened in tiles against the current root; the
+ * whole row, for binary32 rows whose K-th value is tied in a way the heap
+ * layout decides (bf16 rows: topk_replay_kernel).  Elements are screened in tiles against the current root; the
  * screened ones (in index order) are inserted by one lane.  On return
  * hv[0..K) / hi[0..K) hold the heap. */
-template <int BLOCK, int DT, typename SH>
-__device__ void heap_replay(const char* row, int vocab, int K, SH& sh, float* hv, int32_t* hi)
+template <int BLOCK, typename SH>
+__device__ void heap_replay_f32(const char* row, int vocab, int K, SH& sh, float* hv, int32_t* hi)
 {
     static_assert(SH::kMcap >= BLOCK, "replay tiles fit the merge area");
     float* qv = reinterpret_cast<float*>(sh.mc);
@@ -106,7 +107,7 @@ __device__ void heap_replay(const char* row, int vocab, int K, SH& sh, float* hv
     __syncthreads();
     for (int base = 0; base < vocab; base += BLOCK) {
         const int e = base + tid;
-        const float x = (e < vocab) ? load_elem<DT>(row, e) : 0.0f;
+        const float x = (e < vocab) ? load_elem<0>(row, e) : 0.0f;
         const float root = hv[0];
         const int take = (e < vocab) && !(x <= root);
         int total;
@@ -231,6 +232,190 @@ __device__ __forceinline__ bool block_fast_select(SH& sh, int M, int K, uint64_t
     const int pos = block_exclusive_scan<BLOCK>(keep ? 1 : 0, sh.scan, tot);
     if (keep) surv[pos] = c;
     return true;
+}
+
+/* What follows the selection: the nsurv survivors in sh.surv (in any order) or,
+ * when `ordered`, in sh.sorted by vocabulary index. */
+template <int BLOCK, typename SH>
+__device__ __forceinline__ void topk_tail(const TopkArgs& a, SH& sh, int row, const g4s_params& rp,
+                                          double u, int nsurv, bool ordered, bool need_row,
+                                          uint32_t flags)
+{
+    constexpr int NW = BLOCK / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    if (nsurv == 0) {
+        if (wid == 0) {
+            if (lane == 0) {
+                st_sys(&a.ids[row], -1);
+                if (a.out.flags)
+                    st_sys(&a.out.flags[row],
+                           flags | (need_row ? G4S_FLAG_ROW_RECOMPUTED : G4S_FLAG_EMPTY));
+                if (a.out.count) a.out.count[row] = 0;
+            }
+            publish_done(a.done, row, a.seq);
+        }
+        return;
+    }
+
+    /* one survivor per thread (nsurv <= K <= BLOCK): its slot in vocab-index
+     * order (given by the small select, else rank by count; indices are
+     * distinct), then the reference's per-survivor steps */
+    const float cap_v = a.softcap;
+    const float T = rp.temperature;
+    const bool scale = (T > 0.0f) && (T != 1.0f);
+    const float inv_t = scale ? div_cr32(1.0f, T) : 1.0f;               /* :2782 */
+    uint32_t kv = 0u;
+    float vv = 0.0f;
+    int pos = 0;
+    /* p's storage holds the rank counters until the tail writes p */
+    uint32_t* rk = reinterpret_cast<uint32_t*>(sh.prob);
+    if (!ordered) {
+        /* rank by count over the whole workgroup: thread (i, s) counts the
+         * survivors of slice s with an index below survivor i's into i's
+         * counter */
+        for (int i = tid; i < nsurv; i += BLOCK) rk[i] = 0u;
+        __syncthreads();
+        const int npad = (nsurv + 63) & ~63; /* <= KCAP <= BLOCK */
+        const int SL = BLOCK / npad;
+        const int i = tid % npad, sl = tid / npad;
+        if (sl < SL && i < nsurv) {
+            const int per = (nsurv + SL - 1) / SL;
+            const int j0 = sl * per, j1 = j0 + per < nsurv ? j0 + per : nsurv;
+            const uint32_t mi = cand_idx_of(sh.surv[i]);
+            uint32_t c = 0u;
+            int j = j0;
+            for (; j + 8 <= j1; j += 8) {
+                uint32_t xx[8];
+#pragma unroll
+                for (int t = 0; t < 8; ++t) xx[t] = cand_idx_of(sh.surv[j + t]);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) c += xx[t] < mi ? 1u : 0u;
+            }
+            for (; j < j1; ++j) c += cand_idx_of(sh.surv[j]) < mi ? 1u : 0u;
+            if (c != 0u) atomicAdd(&rk[i], c);
+        }
+        __syncthreads();
+    }
+    if (tid < nsurv) {
+        uint64_t my;
+        if (ordered) {
+            pos = tid;
+            my = sh.sorted[tid];
+        } else {
+            my = sh.surv[tid];
+            pos = (int)rk[tid];
+            sh.sorted[pos] = my;
+        }
+        const float x = key2f(cand_key_of(my));                         /* :2774 */
+        vv = (cap_v > 0.0f) ? softcap_topk_cr32(x, cap_v) : x;          /* :2775-2776 */
+        if (scale) vv = vv * inv_t;                                     /* :2783-2784 */
+        kv = f2key(vv);
+    }
+    kv = wave_max_u32(kv);
+    if (lane == 0) sh.red[wid] = kv;
+    __syncthreads();
+    uint32_t kmax = 0u;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) kmax = g4s_max_u(kmax, sh.red[w]);
+    const float vmax = key2f(kmax);                                     /* :2789-2792 */
+    if (tid < nsurv) sh.val[pos] = exp_diff_cr32(vv, vmax);             /* :2797 */
+    const int npad = (nsurv + 63) & ~63; /* <= KCAP, a multiple of 64 */
+    if (tid >= nsurv && tid < npad) {
+        sh.val[tid] = 0.0f;
+        sh.prob[tid] = 0.0f;
+    }
+    __syncthreads();
+
+    /* ------------------------------------------------ tail (wave 0 only) */
+    if (wid != 0) return;
+    /* LSum := LSum + LVals[LI], left to right in binary32 (:2798), every
+     * lane on the same broadcast LDS reads; the padding adds +0, which
+     * leaves a non-negative sum unchanged */
+    float lsum = 0.0f;
+    for (int base = 0; base < npad; base += 64) {
+        const float4* src = reinterpret_cast<const float4*>(sh.val + base);
+#pragma unroll
+        for (int l4 = 0; l4 < 16; ++l4) {
+            const float4 x = src[l4];
+            lsum = lsum + x.x;
+            lsum = lsum + x.y;
+            lsum = lsum + x.z;
+            lsum = lsum + x.w;
+        }
+    }
+    /* greedy choice: first position of the largest p (p >= 0, so its bits
+     * order like the values) */
+    uint32_t pbest = 0u;
+    int jbest = 0x7FFFFFFF;
+    for (int j = lane; j < nsurv; j += 64) {
+        const float p = div_cr32(sh.val[j], lsum);                      /* :2800-2801 */
+        sh.prob[j] = p;
+        if (__float_as_uint(p) > pbest || jbest == 0x7FFFFFFF) {
+            pbest = __float_as_uint(p);
+            jbest = j;
+        }
+    }
+    const uint32_t pmax = wave_max_u32(jbest == 0x7FFFFFFF ? 0u : pbest); /* :2804-2807 */
+    const int jarg =
+        (int)wave_min_u32((jbest != 0x7FFFFFFF && pbest == pmax) ? (uint32_t)jbest : 0xFFFFFFFFu);
+    __builtin_amdgcn_wave_barrier();
+    int chosen = jarg;
+    if (T > 0.0f) {                                                     /* :2811-2824 */
+        flags |= G4S_FLAG_DREW;
+        const float thr = mul_u_p_cr32(u, rp.top_p);
+        /* LCum := LCum + LVals[LI] left to right (broadcast LDS reads as
+         * for LSum); every running sum goes back to LDS (the e values are no
+         * longer needed), then lane l reads the one after term base + l and
+         * one ballot finds the first that reaches thr (a +0 padding term
+         * leaves the sum unchanged, so it never reaches thr first) */
+        float cum = 0.0f;
+        int hit = -1;
+        __builtin_amdgcn_wave_barrier();
+        for (int base = 0; base < npad; base += 64) {
+            const float4* src = reinterpret_cast<const float4*>(sh.prob + base);
+            float4* dst = reinterpret_cast<float4*>(sh.val + base);
+#pragma unroll
+            for (int l4 = 0; l4 < 16; ++l4) {
+                const float4 x = src[l4];
+                float4 c;
+                cum = cum + x.x;
+                c.x = cum;
+                cum = cum + x.y;
+                c.y = cum;
+                cum = cum + x.z;
+                c.z = cum;
+                cum = cum + x.w;
+                c.w = cum;
+                dst[l4] = c; /* the same value from every lane */
+            }
+            __builtin_amdgcn_wave_barrier();
+            const uint64_t reach = __ballot(sh.val[base + lane] >= thr);
+            if (reach) {
+                hit = base + (int)__builtin_ctzll(reach);
+                break;
+            }
+        }
+        if (hit >= 0) {
+            chosen = hit;
+            flags |= G4S_FLAG_REACHED;
+        }
+    }
+    if (lane == 0) {
+        st_sys(&a.ids[row], (int32_t)cand_idx_of(sh.sorted[chosen]));   /* :2826 */
+        if (a.out.count) a.out.count[row] = nsurv;
+        if (a.out.argmax) a.out.argmax[row] = (int32_t)cand_idx_of(sh.sorted[jarg]);
+        if (a.out.lsum) a.out.lsum[row] = lsum;
+        if (a.out.flags) st_sys(&a.out.flags[row], flags);
+    }
+    if (a.out.indices || a.out.probs) {
+        const int capn = a.out.capacity < nsurv ? a.out.capacity : nsurv;
+        for (int j = lane; j < capn; j += 64) {
+            if (a.out.indices)
+                a.out.indices[(int64_t)row * a.out.capacity + j] = (int32_t)cand_idx_of(sh.sorted[j]);
+            if (a.out.probs) a.out.probs[(int64_t)row * a.out.capacity + j] = sh.prob[j];
+        }
+    }
+    publish_done(a.done, row, a.seq);
 }
 
 }  // namespace
@@ -606,6 +791,7 @@ __global__ __launch_bounds__(BLOCK) void topk_kernel(TopkArgs a)
 
     /* exact top K of the M candidates */
     int nsurv = 0;
+    bool pending = false; /* left to topk_replay_kernel */
     bool general = any_exact || M > MCAP;
     bool ordered = false; /* survivors already in sh.sorted by index */
     if (!general && K == 1 && M > 1) {
@@ -774,10 +960,12 @@ __global__ __launch_bounds__(BLOCK) void topk_kernel(TopkArgs a)
                 nsurv = sv;
             } else if (!a.logits) {
                 need_row = true; /* the replay needs every logit */
+            } else if constexpr (DT == 1) {
+                pending = true;
             } else {
                 float* hv = reinterpret_cast<float*>(sh.surv);
                 int32_t* hi = reinterpret_cast<int32_t*>(sh.surv) + KCAP;
-                heap_replay<BLOCK, DT>(rowp, V, K, sh, hv, hi);
+                heap_replay_f32<BLOCK>(rowp, V, K, sh, hv, hi);
                 /* the heap holds K entries, all with index >= 0 here (M > K);
                  * K <= kbound <= BLOCK, so one entry per thread */
                 uint64_t mine_e = 0;
@@ -790,179 +978,48 @@ __global__ __launch_bounds__(BLOCK) void topk_kernel(TopkArgs a)
     }
     __syncthreads();
 
-    if (nsurv == 0) {
-        if (wid == 0) {
-            if (lane == 0) {
-                st_sys(&a.ids[row], -1);
-                if (a.out.flags)
-                    st_sys(&a.out.flags[row],
-                           flags | (need_row ? G4S_FLAG_ROW_RECOMPUTED : G4S_FLAG_EMPTY));
-                if (a.out.count) a.out.count[row] = 0;
-            }
-            publish_done(a.done, row, a.seq);
-        }
-        return;
+    if constexpr (DT == 1) {
+        if (tid == 0) st_dev(&a.wbounds[(int64_t)row * kWaveBounds], pending ? flags : 0u);
+        if (pending) return;
     }
+    topk_tail<BLOCK>(a, sh, row, rp, u, nsurv, ordered, need_row, flags);
+}
 
-    /* one survivor per thread (nsurv <= K <= BLOCK): its slot in vocab-index
-     * order (given by the small select, else rank by count; indices are
-     * distinct), then the reference's per-survivor steps */
-    const float cap_v = a.softcap;
-    const float T = rp.temperature;
-    const bool scale = (T > 0.0f) && (T != 1.0f);
-    const float inv_t = scale ? div_cr32(1.0f, T) : 1.0f;               /* :2782 */
-    uint32_t kv = 0u;
-    float vv = 0.0f;
-    int pos = 0;
-    /* p's storage holds the rank counters until the tail writes p */
-    uint32_t* rk = reinterpret_cast<uint32_t*>(sh.prob);
-    if (!ordered) {
-        /* rank by count over the whole workgroup: thread (i, s) counts the
-         * survivors of slice s with an index below survivor i's into i's
-         * counter */
-        for (int i = tid; i < nsurv; i += BLOCK) rk[i] = 0u;
-        __syncthreads();
-        const int npad = (nsurv + 63) & ~63; /* <= KCAP <= BLOCK */
-        const int SL = BLOCK / npad;
-        const int i = tid % npad, sl = tid / npad;
-        if (sl < SL && i < nsurv) {
-            const int per = (nsurv + SL - 1) / SL;
-            const int j0 = sl * per, j1 = j0 + per < nsurv ? j0 + per : nsurv;
-            const uint32_t mi = cand_idx_of(sh.surv[i]);
-            uint32_t c = 0u;
-            int j = j0;
-            for (; j + 8 <= j1; j += 8) {
-                uint32_t xx[8];
-#pragma unroll
-                for (int t = 0; t < 8; ++t) xx[t] = cand_idx_of(sh.surv[j + t]);
-#pragma unroll
-                for (int t = 0; t < 8; ++t) c += xx[t] < mi ? 1u : 0u;
-            }
-            for (; j < j1; ++j) c += cand_idx_of(sh.surv[j]) < mi ? 1u : 0u;
-            if (c != 0u) atomicAdd(&rk[i], c);
-        }
-        __syncthreads();
-    }
-    if (tid < nsurv) {
-        uint64_t my;
-        if (ordered) {
-            pos = tid;
-            my = sh.sorted[tid];
-        } else {
-            my = sh.surv[tid];
-            pos = (int)rk[tid];
-            sh.sorted[pos] = my;
-        }
-        const float x = key2f(cand_key_of(my));                         /* :2774 */
-        vv = (cap_v > 0.0f) ? softcap_topk_cr32(x, cap_v) : x;          /* :2775-2776 */
-        if (scale) vv = vv * inv_t;                                     /* :2783-2784 */
-        kv = f2key(vv);
-    }
-    kv = wave_max_u32(kv);
-    if (lane == 0) sh.red[wid] = kv;
-    __syncthreads();
-    uint32_t kmax = 0u;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) kmax = g4s_max_u(kmax, sh.red[w]);
-    const float vmax = key2f(kmax);                                     /* :2789-2792 */
-    if (tid < nsurv) sh.val[pos] = exp_diff_cr32(vv, vmax);             /* :2797 */
-    const int npad = (nsurv + 63) & ~63; /* <= KCAP, a multiple of 64 */
-    if (tid >= nsurv && tid < npad) {
-        sh.val[tid] = 0.0f;
-        sh.prob[tid] = 0.0f;
-    }
-    __syncthreads();
+constexpr int kReplayBlock = 1024;
+constexpr int kReplayQueue = 4096;
 
-    /* ------------------------------------------------ tail (wave 0 only) */
-    if (wid != 0) return;
-    /* LSum := LSum + LVals[LI], left to right in binary32 (:2798), every
-     * lane on the same broadcast LDS reads; the padding adds +0, which
-     * leaves a non-negative sum unchanged */
-    float lsum = 0.0f;
-    for (int base = 0; base < npad; base += 64) {
-        const float4* src = reinterpret_cast<const float4*>(sh.val + base);
-#pragma unroll
-        for (int l4 = 0; l4 < 16; ++l4) {
-            const float4 x = src[l4];
-            lsum = lsum + x.x;
-            lsum = lsum + x.y;
-            lsum = lsum + x.z;
-            lsum = lsum + x.w;
-        }
-    }
-    /* greedy choice: first position of the largest p (p >= 0, so its bits
-     * order like the values) */
-    uint32_t pbest = 0u;
-    int jbest = 0x7FFFFFFF;
-    for (int j = lane; j < nsurv; j += 64) {
-        const float p = div_cr32(sh.val[j], lsum);                      /* :2800-2801 */
-        sh.prob[j] = p;
-        if (__float_as_uint(p) > pbest || jbest == 0x7FFFFFFF) {
-            pbest = __float_as_uint(p);
-            jbest = j;
-        }
-    }
-    const uint32_t pmax = wave_max_u32(jbest == 0x7FFFFFFF ? 0u : pbest); /* :2804-2807 */
-    const int jarg =
-        (int)wave_min_u32((jbest != 0x7FFFFFFF && pbest == pmax) ? (uint32_t)jbest : 0xFFFFFFFFu);
-    __builtin_amdgcn_wave_barrier();
-    int chosen = jarg;
-    if (T > 0.0f) {                                                     /* :2811-2824 */
-        flags |= G4S_FLAG_DREW;
-        const float thr = mul_u_p_cr32(u, rp.top_p);
-        /* LCum := LCum + LVals[LI] left to right (broadcast LDS reads as
-         * for LSum); every running sum goes back to LDS (the e values are no
-         * longer needed), then lane l reads the one after term base + l and
-         * one ballot finds the first that reaches thr (a +0 padding term
-         * leaves the sum unchanged, so it never reaches thr first) */
-        float cum = 0.0f;
-        int hit = -1;
-        __builtin_amdgcn_wave_barrier();
-        for (int base = 0; base < npad; base += 64) {
-            const float4* src = reinterpret_cast<const float4*>(sh.prob + base);
-            float4* dst = reinterpret_cast<float4*>(sh.val + base);
-#pragma unroll
-            for (int l4 = 0; l4 < 16; ++l4) {
-                const float4 x = src[l4];
-                float4 c;
-                cum = cum + x.x;
-                c.x = cum;
-                cum = cum + x.y;
-                c.y = cum;
-                cum = cum + x.z;
-                c.z = cum;
-                cum = cum + x.w;
-                c.w = cum;
-                dst[l4] = c; /* the same value from every lane */
-            }
-            __builtin_amdgcn_wave_barrier();
-            const uint64_t reach = __ballot(sh.val[base + lane] >= thr);
-            if (reach) {
-                hit = base + (int)__builtin_ctzll(reach);
-                break;
-            }
-        }
-        if (hit >= 0) {
-            chosen = hit;
-            flags |= G4S_FLAG_REACHED;
-        }
-    }
-    if (lane == 0) {
-        st_sys(&a.ids[row], (int32_t)cand_idx_of(sh.sorted[chosen]));   /* :2826 */
-        if (a.out.count) a.out.count[row] = nsurv;
-        if (a.out.argmax) a.out.argmax[row] = (int32_t)cand_idx_of(sh.sorted[jarg]);
-        if (a.out.lsum) a.out.lsum[row] = lsum;
-        if (a.out.flags) st_sys(&a.out.flags[row], flags);
-    }
-    if (a.out.indices || a.out.probs) {
-        const int capn = a.out.capacity < nsurv ? a.out.capacity : nsurv;
-        for (int j = lane; j < capn; j += 64) {
-            if (a.out.indices)
-                a.out.indices[(int64_t)row * a.out.capacity + j] = (int32_t)cand_idx_of(sh.sorted[j]);
-            if (a.out.probs) a.out.probs[(int64_t)row * a.out.capacity + j] = sh.prob[j];
-        }
-    }
-    publish_done(a.done, row, a.seq);
+/* The rows that the launch before left to a replay of the heap (bf16 logits:
+ * nearly every row, ties being ordinary there): one workgroup per row, the
+ * other rows' end at once (a synchronous call without ties takes 25.6 us with
+ * and without this launch).  Inlined in the kernels that find the tie, the
+ * replay takes registers from every row (64 mixed binary32 rows 37.5 -> 38.6
+ * us); binary32 rows tie rarely and keep the serial one in place. */
+template <int DT>
+__global__ __launch_bounds__(kReplayBlock) void topk_replay_kernel(TopkArgs a)
+{
+    __shared__ TopkShared<kMaxTopK, 64> sh;
+    __shared__ alignas(16) uint64_t heap[kMaxTopK + kHeapExtra];
+    __shared__ uint64_t q[kReplayQueue];
+    __shared__ HeapCtl ctl;
+    const int tid = threadIdx.x;
+    const int row = blockIdx.x;
+    const g4s_params rp = a.params ? a.params[row] : a.p0;
+    const double u = a.u ? a.u[row] : a.u0;
+    const int K = rp.top_k;
+    if (!(K >= 1 && K < a.vocab) || K > a.kbound) return; /* no top-k row */
+    const uint32_t flags = a.wbounds[(int64_t)row * kWaveBounds];
+    if (flags == 0u) return;
+    const char* rowp = reinterpret_cast<const char*>(a.logits) +
+                       (int64_t)row * a.row_stride * Elem<DT>::SIZE;
+    heap_replay<kReplayBlock, DT>(rowp, a.vocab, K, heap, q, kReplayQueue, ctl);
+    /* the entries holding an index survive (Model.pas:2668-2676) */
+    const uint64_t e = tid < K ? heap[tid + 1] : heap_pack(0.0f, -1);
+    const bool valid = heap_idx(e) >= 0;
+    int nsurv;
+    const int at = block_exclusive_scan<kReplayBlock>(valid ? 1 : 0, sh.scan, nsurv);
+    if (valid) sh.surv[at] = cand_pack(f2key(heap_val(e)), (uint32_t)heap_idx(e));
+    __syncthreads();
+    topk_tail<kReplayBlock>(a, sh, row, rp, u, nsurv, false, false, flags);
 }
 
 /* ------------------------------------- candidates from 64-row group maxima */
@@ -1509,8 +1566,8 @@ hipError_t topk_groups_launch(const TopkConfig& c, const TopkArgs& a, const uint
     return launch_one<1024, 64, 0>(b, a.kbound, s);
 }
 
-hipError_t topk_launch(const TopkConfig& c, const TopkArgs& a, int dtype, hipStream_t s,
-                       int32_t ncu)
+static hipError_t topk_select_launch(const TopkConfig& c, const TopkArgs& a, int dtype,
+                                     hipStream_t s, int32_t ncu)
 {
     if (decode_eligible(a, dtype)) return decode_launch(a, dtype, s);
     const int kc = a.kbound;
@@ -1522,6 +1579,19 @@ hipError_t topk_launch(const TopkConfig& c, const TopkArgs& a, int dtype, hipStr
     if (c.block == 512 && c.items == 16) return launch_cfg<512, 16, 1>(a, kc, s, ncu);
     if (c.block == 1024 && c.items == 32) return launch_cfg<1024, 32, 1>(a, kc, s, ncu);
     return launch_cfg<1024, 64, 1>(a, kc, s, ncu);
+}
+
+hipError_t topk_launch(const TopkConfig& c, const TopkArgs& a, int dtype, hipStream_t s,
+                       int32_t ncu)
+{
+    hipError_t e = topk_select_launch(c, a, dtype, s, ncu);
+    /* K = 1 keeps the first copy of the largest key: no replay */
+    if (e == hipSuccess && dtype == G4S_DTYPE_BF16 && a.kbound > 1) {
+        hipLaunchKernelGGL(topk_replay_kernel<1>, dim3((unsigned)a.batch), dim3(kReplayBlock), 0, s,
+                           a);
+        e = hipGetLastError();
+    }
+    return e;
 }
 
 }  // namespace g4s
