@@ -151,6 +151,11 @@ struct FullWorkspace {
     uint32_t* bits = nullptr;    /* [max_batch][ceil(vocab/32)] surviving tied copies */
     uint64_t* heap = nullptr;    /* [vocab + kHeapExtra] replay heap of rows that LDS does not
                                     hold (one row at a time) */
+    /* e of every term of the first erows rows of a binary32 launch, written by the
+     * LSum pass and read by what follows ([erows][cstride * kFullChunk]; -0: the
+     * term does not take part) */
+    float* eterm = nullptr;
+    int32_t erows = 0;
     /* streaming pipeline of full bf16 rows */
     float* ytab = nullptr;       /* [65536] y = softcap(x) of every bf16 code (full-row form) */
     FbRow* fbrow = nullptr;      /* [max_batch] */
@@ -177,6 +182,7 @@ struct FullArgs {
     int32_t nsel;     /* chunks of kSelChunk terms per row (wide select) */
     int32_t nstage;   /* chunks each chain precomputes (set by full_launch) */
     int32_t cpw;      /* chunks per wave of the streaming passes (set by full_launch) */
+    int32_t row0;     /* first row of a launch over a part of the batch (set by full_launch) */
     int32_t wide_on;  /* wide rows are handled by this launch */
     int32_t topk_on;  /* a top-k launch takes the top-k rows; when 0 such a row gets
                          id -1 and G4S_FLAG_ERROR | G4S_FLAG_TOPK_PATH here */

@@ -43,7 +43,8 @@
  *             the streaming passes look e up; the predicted binade of LSum
  *             entering every chunk (a parallel prefix of the estimates);
  *   3 lsum:   each chunk's terms as one exact map of the running sum in its
- *             predicted binade (g4s_seqsum.h);
+ *             predicted binade (g4s_seqsum.h); binary32 rows keep their terms
+ *             in device memory for 4 to 6;
  *   4 chain:  LSum: the workgroup stages in LDS the chunks where the sum is
  *             predicted to change binade, then wave 0 composes the chunk
  *             maps 64 at a time, verifying every step, and re-evaluates the
@@ -593,6 +594,49 @@ struct TabLds {
     float tab[DT == 1 ? kFullTab : 1];
 };
 
+/* Lane l's 16 terms of a chunk held in LDS in index order. */
+__device__ __forceinline__ void lds_terms(const float* sh, float (&t)[kFullPer])
+{
+    const float4* src = reinterpret_cast<const float4*>(sh + (threadIdx.x & 63) * kFullPer);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float4 v = src[q];
+        t[4 * q] = v.x;
+        t[4 * q + 1] = v.y;
+        t[4 * q + 2] = v.z;
+        t[4 * q + 3] = v.w;
+    }
+}
+
+/* A wave's terms with e = 1 - jj*2^-24, jj < kNear (the row maximum and its
+ * near ties): looked at only in waves that hold one.  The first index of e ==
+ * 1 and, on wide rows, of each near tie. */
+__device__ __forceinline__ void near_ties(const float (&t)[kFullPer], int64_t e0, const Mask& k,
+                                          FullRow* rr)
+{
+    const int lane = threadIdx.x & 63;
+    constexpr float kNearLo = 1.0f - (float)(kNear - 1) * 0x1p-24f;
+    float tmx = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kFullPer; ++j) tmx = __builtin_fmaxf(tmx, t[j]);
+    if (__ballot(tmx >= kNearLo)) {
+        uint32_t first1 = 0xFFFFFFFFu;
+        uint32_t nearm = 0u;
+#pragma unroll
+        for (int j = 0; j < kFullPer; ++j) {
+            first1 = t[j] == 1.0f ? g4s_min_u(first1, (uint32_t)(e0 + j)) : first1;
+            nearm |= (t[j] >= kNearLo && t[j] < 1.0f) ? (1u << j) : 0u;
+        }
+        if (k.cls == kRowWide && nearm != 0u) {
+            for (int j = 0; j < kFullPer; ++j)
+                if (nearm & (1u << j))
+                    atomicMin(&rr->near[(int)((1.0f - t[j]) * 0x1p24f)], (int32_t)(e0 + j));
+        }
+        first1 = wave_min_u32(first1);
+        if (lane == 0 && first1 != 0xFFFFFFFFu) atomicMin(&rr->near[0], (int32_t)first1);
+    }
+}
+
 /* Each chunk's terms as one map of LSum in the chunk's predicted binade,
  * one chunk per wave at a time; the first index of e == 1 and, on wide rows,
  * of its near ties. */
@@ -601,7 +645,7 @@ __global__ __launch_bounds__(kFullBlock) void full_lsum_kernel(FullArgs a)
 {
     __shared__ TabLds<DT> sh;
     const int lane = threadIdx.x & 63;
-    const int row = blockIdx.y;
+    const int row = a.row0 + blockIdx.y;
     const int V = a.vocab;
     const int nch = a.nch;
     if ((int)blockIdx.x * NWF * a.cpw >= nch) return;
@@ -633,34 +677,57 @@ __global__ __launch_bounds__(kFullBlock) void full_lsum_kernel(FullArgs a)
             nvalid = load16<DT>(rowp, e0, V, raw);
             tabbed = terms_e<DT>(raw, nvalid, e0, c, k, sh.tab, t);
         }
-        /* the terms with e = 1 - jj*2^-24, jj < kNear (the row maximum and
-         * its near ties): looked at only in waves that hold one */
-        constexpr float kNearLo = 1.0f - (float)(kNear - 1) * 0x1p-24f;
-        float tmx = 0.0f;
-#pragma unroll
-        for (int j = 0; j < kFullPer; ++j) tmx = __builtin_fmaxf(tmx, t[j]);
-        if (__ballot(tmx >= kNearLo)) {
-            uint32_t first1 = 0xFFFFFFFFu;
-            uint32_t nearm = 0u;
-#pragma unroll
-            for (int j = 0; j < kFullPer; ++j) {
-                first1 = t[j] == 1.0f ? g4s_min_u(first1, (uint32_t)(e0 + j)) : first1;
-                nearm |= (t[j] >= kNearLo && t[j] < 1.0f) ? (1u << j) : 0u;
-            }
-            if (k.cls == kRowWide && nearm != 0u) {
-                for (int j = 0; j < kFullPer; ++j)
-                    if (nearm & (1u << j))
-                        atomicMin(&rr->near[(int)((1.0f - t[j]) * 0x1p24f)], (int32_t)(e0 + j));
-            }
-            first1 = wave_min_u32(first1);
-            if (lane == 0 && first1 != 0xFFFFFFFFu) atomicMin(&rr->near[0], (int32_t)first1);
-        }
+        near_ties(t, e0, k, rr);
         const int32_t beta = __builtin_amdgcn_readlane(betas, b - cw);
         const PMap cm = wave_chunk_map(tabbed && !tie_possible(tm, kTieBaseE, beta)
                                            ? thread_map_nt(t, beta)
                                            : thread_map(t, nvalid, beta));
         if (lane == 0) a.ws.lmap[rbase + b] = cm;
     }
+}
+
+/* binary32 rows whose terms are kept (a.ws.eterm): one workgroup per chunk,
+ * four terms per thread, and the chunk's map by its first wave.  The correctly
+ * rounded softcap and exp are a chain of about 150 dependent binary64
+ * operations a term: at 16 terms a lane one row is 256 waves of 16 chains each
+ * (16.7 us, here 7.8; 24 rows of 100,003 22.8 us, here 16.7).  Kept, the terms
+ * are not evaluated again by the draw's pass (18.9 -> 5.1 us, 37.3 -> 8.5) and
+ * by the staged chunks of the two chains (38.4 and 41.2 -> 25 us each).  The
+ * 100th row of a batch is beyond them: such rows take full_lsum_kernel. */
+static_assert(kFullBlock * 4 == kFullChunk, "four terms per thread");
+__global__ __launch_bounds__(kFullBlock) void full_lsum_store_kernel(FullArgs a)
+{
+    __shared__ alignas(16) float sh[kFullChunk];
+    const int tid = threadIdx.x;
+    const int row = blockIdx.y, b = blockIdx.x;
+    const RowIn ri = row_in(a, row);
+    Mask k;
+    if (!row_mask(a, row, ri, k)) return;
+    FullRow* rr = a.ws.rows + row;
+    const FullRow r = *rr;
+    const Ctx c = make_ctx(a, r, k.cls);
+    const int64_t e4 = (int64_t)b * kFullChunk + tid * 4;
+    float x[4];
+    load_vec<0>(row_ptr<0>(a, row), e4, a.vocab, x);
+    float e[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const bool part = e4 + j < a.vocab && takes_part(k, x[j], e4 + j);
+        e[j] = part ? e_direct(x[j], c) : -0.0f;                       /* Tensors.pas:660 */
+    }
+    float* et = a.ws.eterm + (int64_t)row * a.ws.cstride * kFullChunk;
+    *reinterpret_cast<float4*>(et + e4) = make_float4(e[0], e[1], e[2], e[3]);
+    *reinterpret_cast<float4*>(sh + tid * 4) =
+        make_float4(term_of<false>(e[0], c), term_of<false>(e[1], c), term_of<false>(e[2], c),
+                    term_of<false>(e[3], c));
+    __syncthreads();
+    if (tid >= 64) return;
+    float t[kFullPer];
+    lds_terms(sh, t);
+    near_ties(t, (int64_t)b * kFullChunk + tid * kFullPer, k, rr);
+    const int64_t at = (int64_t)row * a.ws.cstride + b;
+    const PMap cm = wave_chunk_map(thread_map(t, kFullPer, a.ws.beta_l[at]));
+    if (tid == 0) a.ws.lmap[at] = cm;
 }
 
 /* ------------------------------------------------------- 4: LSum chain */
@@ -713,7 +780,7 @@ __global__ __launch_bounds__(kChainBlock) void full_lsum_chain_kernel(FullArgs a
             }
             ++reev;
             int h;
-            st = chain_chunk<DT, false>(a, rowp, cb, st, __builtin_inff(), L, c, k, r, &h, &rounds);
+            st = chain_chunk<DT, false>(a, rowp, stored_row<DT>(a, row), cb, st, __builtin_inff(), L, c, k, r, &h, &rounds);
             if (lane == 0) L.cpost[cb] = ss::value_of(st);
             ++cb;
         }
@@ -803,7 +870,7 @@ __global__ __launch_bounds__(kFullBlock) void full_cdf_kernel(FullArgs a)
 {
     __shared__ TabLds<DT> sh;
     const int lane = threadIdx.x & 63;
-    const int row = blockIdx.y;
+    const int row = a.row0 + blockIdx.y;
     const int V = a.vocab;
     const RowIn ri = row_in(a, row);
     Mask k;
@@ -876,6 +943,65 @@ __global__ __launch_bounds__(kFullBlock) void full_cdf_kernel(FullArgs a)
     }
 }
 
+/* The same for rows whose terms are kept: p from the stored e, one workgroup
+ * per chunk up to the row's last draw chunk. */
+__global__ __launch_bounds__(kFullBlock) void full_cdf_store_kernel(FullArgs a)
+{
+    __shared__ alignas(16) float sh[kFullChunk];
+    __shared__ Scratch sc;
+    const int tid = threadIdx.x;
+    const int row = blockIdx.y, b = blockIdx.x;
+    const RowIn ri = row_in(a, row);
+    Mask k;
+    if (!row_mask(a, row, ri, k)) return;
+    const FullRow r = a.ws.rows[row];
+    if (b > r.c_last) return;
+    const Ctx c = make_ctx(a, r, k.cls);
+    const int64_t at = (int64_t)row * a.ws.cstride + b;
+    const int64_t e4 = (int64_t)b * kFullChunk + tid * 4;
+    const float4 ev = *reinterpret_cast<const float4*>(stored_row<0>(a, row) + e4);
+    const float e[4] = {ev.x, ev.y, ev.z, ev.w};
+    float p[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p[j] = term_of<true>(e[j], c);
+    if (term_outputs(a, k.cls)) {
+        float* po = a.out.probs ? a.out.probs + (int64_t)row * a.out.capacity : nullptr;
+        int32_t* io = a.out.indices ? a.out.indices + (int64_t)row * a.out.capacity : nullptr;
+        if (k.cls == kRowFull) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (e4 + j < a.vocab) {
+                    po[e4 + j] = p[j]; /* Tensors.pas:671 */
+                    if (io) io[e4 + j] = (int32_t)(e4 + j);
+                }
+        } else {
+            /* the survivors in index order (Model.pas:2678-2688) */
+            int cnt = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) cnt += __float_as_uint(e[j]) != 0x80000000u ? 1 : 0;
+            int total;
+            int pos = a.ws.chunks[at].soff + block_excl_scan_i(cnt, sc, total);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (__float_as_uint(e[j]) != 0x80000000u) {
+                    if (pos < a.out.capacity) {
+                        if (po) po[pos] = p[j];
+                        if (io) io[pos] = (int32_t)(e4 + j);
+                    }
+                    ++pos;
+                }
+        }
+    }
+    if (r.nodraw) return;
+    *reinterpret_cast<float4*>(sh + tid * 4) = make_float4(p[0], p[1], p[2], p[3]);
+    __syncthreads();
+    if (tid >= 64) return;
+    float t[kFullPer];
+    lds_terms(sh, t);
+    const PMap cm = wave_chunk_map(thread_map(t, kFullPer, a.ws.beta_c[at]));
+    if (tid == 0) a.ws.cmap[at] = cm;
+}
+
 /* -------------------------------------------------------- 6: the draw */
 
 /* One workgroup per row: the first index whose left-to-right binary32
@@ -933,7 +1059,7 @@ __global__ __launch_bounds__(kChainBlock) void full_cdf_chain_kernel(FullArgs a)
         }
         ++reev;
         int h;
-        st = chain_chunk<DT, true>(a, rowp, cb, st, thr, L, c, k, r, &h, &rounds);
+        st = chain_chunk<DT, true>(a, rowp, stored_row<DT>(a, row), cb, st, thr, L, c, k, r, &h, &rounds);
         if (h >= 0) {
             hit = (int64_t)cb * kFullChunk + h;
             break;
@@ -960,6 +1086,10 @@ bool full_supported(int32_t vocab)
            (vocab + kSelChunk - 1) / kSelChunk <= kSelMaxChunks;
 }
 
+/* Terms kept per handle: 64 rows of 262,144 (a bound on what a handle of many
+ * rows takes; a hundred such rows 347 -> 321 us, 64 rows 253 -> 160). */
+constexpr size_t kEtermBytes = (size_t)64 << 20;
+
 hipError_t full_alloc(FullWorkspace& ws, int32_t vocab, int32_t max_batch)
 {
     const size_t mb = (size_t)max_batch;
@@ -968,12 +1098,15 @@ hipError_t full_alloc(FullWorkspace& ws, int32_t vocab, int32_t max_batch)
     const size_t nc = mb * (size_t)ws.cstride;
     hipError_t e = hipMalloc((void**)&ws.rows, mb * sizeof(FullRow));
     if (e == hipSuccess) e = hipMalloc((void**)&ws.chunks, nc * sizeof(FullChunk));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.lmap, nc * sizeof(PMap));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.cmap, nc * sizeof(PMap));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.beta_l, nc * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.beta_c, nc * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.etab, mb * kFullTab * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.ptab, mb * kFullTab * sizeof(float));
+    /* the two maps, binades and tables share an allocation each */
+    if (e == hipSuccess) e = hipMalloc((void**)&ws.lmap, 2 * nc * sizeof(PMap));
+    if (e == hipSuccess) e = hipMalloc((void**)&ws.beta_l, 2 * nc * sizeof(int32_t));
+    if (e == hipSuccess) e = hipMalloc((void**)&ws.etab, 2 * mb * kFullTab * sizeof(float));
+    if (e == hipSuccess) {
+        ws.cmap = ws.lmap + nc;
+        ws.beta_c = ws.beta_l + nc;
+        ws.ptab = ws.etab + mb * kFullTab;
+    }
     if (e == hipSuccess) e = hipMalloc((void**)&ws.tmask, mb * 2 * sizeof(uint64_t));
     if (e == hipSuccess) e = hipMalloc((void**)&ws.sel, mb * sizeof(WideSel));
     if (e == hipSuccess) e = hipMalloc((void**)&ws.hist, mb * kWideBins * sizeof(uint32_t));
@@ -982,6 +1115,17 @@ hipError_t full_alloc(FullWorkspace& ws, int32_t vocab, int32_t max_batch)
         e = hipMalloc((void**)&ws.bits, mb * (size_t)ws.bits_stride * sizeof(uint32_t));
     if (e == hipSuccess)
         e = hipMalloc((void**)&ws.heap, ((size_t)vocab + kHeapExtra) * sizeof(uint64_t));
+    if (e == hipSuccess) {
+        /* without it (or beyond it) the passes evaluate the terms again */
+        const size_t per = (size_t)ws.cstride * kFullChunk * sizeof(float);
+        const size_t rows = kEtermBytes / per;
+        ws.erows = (int32_t)(rows < mb ? rows : mb);
+        if (ws.erows && hipMalloc((void**)&ws.eterm, ws.erows * per) != hipSuccess) {
+            (void)hipGetLastError();
+            ws.eterm = nullptr;
+            ws.erows = 0;
+        }
+    }
     if (e == hipSuccess) e = hipMalloc((void**)&ws.ytab, (size_t)65536 * sizeof(float));
     if (e == hipSuccess) e = hipMalloc((void**)&ws.fbrow, mb * sizeof(FbRow));
     if (e == hipSuccess) e = hipMalloc((void**)&ws.etab8, mb * kBfTab * sizeof(float));
@@ -994,8 +1138,8 @@ hipError_t full_alloc(FullWorkspace& ws, int32_t vocab, int32_t max_batch)
 
 void full_free(FullWorkspace& ws)
 {
-    void* ptrs[] = {ws.rows, ws.chunks, ws.lmap, ws.cmap, ws.beta_l, ws.beta_c, ws.etab, ws.ptab, ws.tmask,
-                    ws.sel, ws.hist, ws.ties, ws.bits, ws.heap, ws.ytab, ws.fbrow,
+    void* ptrs[] = {ws.rows, ws.chunks, ws.lmap, ws.beta_l, ws.etab, ws.tmask, ws.sel, ws.hist,
+                    ws.ties, ws.bits, ws.heap, ws.eterm, ws.ytab, ws.fbrow,
                     ws.etab8, ws.ptab8, ws.stage, ws.cpost, ws.head};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -1078,6 +1222,7 @@ static hipError_t launch_dt(const FullArgs& a0, hipStream_t s)
     size_t lds = 0;
     a.nstage = chain_nstage<DT>(a.nch, &lds);
     a.cpw = stream_cpw(a.nch, a.batch);
+    a.row0 = 0;
     const dim3 sel((unsigned)a.nsel, (unsigned)a.batch);
     const dim3 rows(1u, (unsigned)a.batch);
     const dim3 waves((unsigned)((a.nch + NWF * a.cpw - 1) / (NWF * a.cpw)), (unsigned)a.batch);
@@ -1096,9 +1241,17 @@ static hipError_t launch_dt(const FullArgs& a0, hipStream_t s)
                        dim3(DT == 1 ? (unsigned)(kFullTab / (kFullBlock * kRowPer)) : 1u,
                             (unsigned)a.batch),
                        dim3(kFullBlock), 0, s, a);
-    hipLaunchKernelGGL((full_lsum_kernel<DT>), waves, dim3(kFullBlock), 0, s, a);
+    /* binary32: the rows whose terms are kept, then any others */
+    const int kept = DT == 0 ? (a.batch < a.ws.erows ? a.batch : a.ws.erows) : 0;
+    const dim3 chunks((unsigned)a.nch, (unsigned)kept);
+    const dim3 rest(waves.x, (unsigned)(a.batch - kept));
+    FullArgs ar = a;
+    ar.row0 = kept;
+    if (kept) hipLaunchKernelGGL(full_lsum_store_kernel, chunks, dim3(kFullBlock), 0, s, a);
+    if (rest.y) hipLaunchKernelGGL((full_lsum_kernel<DT>), rest, dim3(kFullBlock), 0, s, ar);
     hipLaunchKernelGGL((full_lsum_chain_kernel<DT>), rows, dim3(kChainBlock), lds, s, a);
-    hipLaunchKernelGGL((full_cdf_kernel<DT>), waves, dim3(kFullBlock), 0, s, a);
+    if (kept) hipLaunchKernelGGL(full_cdf_store_kernel, chunks, dim3(kFullBlock), 0, s, a);
+    if (rest.y) hipLaunchKernelGGL((full_cdf_kernel<DT>), rest, dim3(kFullBlock), 0, s, ar);
     hipLaunchKernelGGL((full_cdf_chain_kernel<DT>), rows, dim3(kChainBlock), lds, s, a);
     return hipGetLastError();
 }

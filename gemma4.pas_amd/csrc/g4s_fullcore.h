@@ -315,6 +315,22 @@ __device__ __forceinline__ bool terms_e(const uint32_t (&raw)[kFullPer], int nva
     return terms_e_t<DT, false, P>(raw, nvalid, e0, c, k, tab, t);
 }
 
+/* The stored terms of a binary32 row (nullptr: evaluated from x). */
+template <int DT>
+__device__ __forceinline__ const float* stored_row(const FullArgs& a, int row)
+{
+    if (DT != 0 || row >= a.ws.erows) return nullptr;
+    return a.ws.eterm + (int64_t)row * a.ws.cstride * kFullChunk;
+}
+
+/* A stored e as the term it stands for: e, or p of it. */
+template <bool P>
+__device__ __forceinline__ float term_of(float e, const Ctx& c)
+{
+    if (__float_as_uint(e) == 0x80000000u) return 0.0f; /* takes no part */
+    return P ? p_of(e, c.cls, c.inv, c.lsum) : e;
+}
+
 /* ------------------------------------------------------ block helpers */
 
 struct Scratch {
@@ -829,13 +845,20 @@ __device__ __forceinline__ ChainLds chain_lds(char* base, int nch, int nstage)
 
 /* The 16 terms (e, or p when P) of lane `lane` in chunk c. */
 template <int DT, bool P>
-__device__ __forceinline__ int chain_load_terms(const FullArgs& a, const char* rowp, int c,
+__device__ __forceinline__ int chain_load_terms(const FullArgs& a, const char* rowp,
+                                                const float* et, int c,
                                                 const Ctx& ctx, const Mask& k, const FullRow& r,
                                                 const float* tab, float (&t)[kFullPer])
 {
     const int lane = threadIdx.x & 63;
     uint32_t raw[kFullPer];
     const int64_t e0 = (int64_t)c * kFullChunk + (int64_t)lane * kFullPer;
+    if (et) {
+        (void)load16<DT>(reinterpret_cast<const char*>(et), e0, a.ws.cstride * kFullChunk, raw);
+#pragma unroll
+        for (int j = 0; j < kFullPer; ++j) t[j] = term_of<P>(__uint_as_float(raw[j]), ctx);
+        return kFullPer;
+    }
     const int nv = load16<DT>(rowp, e0, a.vocab, raw);
     (void)r;
     terms_e<DT, P>(raw, nv, e0, ctx, k, tab, t);
@@ -928,7 +951,8 @@ __device__ void chain_prologue(const FullArgs& a, int row, const FullRow& r, con
     /* wave w precomputes slot w */
     constexpr int kSlots = kStageMax / kChainWaves;
     constexpr int kVec = kFullPer * Elem<DT>::SIZE / 16; /* 16-byte loads per lane per chunk */
-    const char* rowp = row_ptr<DT>(a, row);
+    const float* et = stored_row<DT>(a, row);
+    const char* rowp = et ? reinterpret_cast<const char*>(et) : row_ptr<DT>(a, row);
     uint4 pk[kSlots][kVec];
     int cs[kSlots];
 #pragma unroll
@@ -963,7 +987,12 @@ __device__ void chain_prologue(const FullArgs& a, int row, const FullRow& r, con
         }
         float t[kFullPer];
         const int64_t e0 = (int64_t)c * kFullChunk + (int64_t)lane * kFullPer;
-        terms_e<DT, P>(raw, kFullPer, e0, ctx, k, L.tab, t);
+        if (et) {
+#pragma unroll
+            for (int j = 0; j < kFullPer; ++j) t[j] = term_of<P>(__uint_as_float(raw[j]), ctx);
+        } else {
+            terms_e<DT, P>(raw, kFullPer, e0, ctx, k, L.tab, t);
+        }
         float4* dst = reinterpret_cast<float4*>(L.tv + (size_t)sl * kFullChunk + lane * kFullPer);
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -986,7 +1015,8 @@ __device__ void chain_prologue(const FullArgs& a, int row, const FullRow& r, con
  * (-1: none).
  */
 template <int DT, bool P>
-__device__ State chain_chunk(const FullArgs& a, const char* rowp, int c, State st, float thr,
+__device__ State chain_chunk(const FullArgs& a, const char* rowp, const float* et, int c,
+                             State st, float thr,
                              const ChainLds& L, const Ctx& ctx, const Mask& k, const FullRow& r,
                              int* hit, int* rounds)
 {
@@ -1025,7 +1055,7 @@ __device__ State chain_chunk(const FullArgs& a, const char* rowp, int c, State s
             }
         }
     } else {
-        nv = chain_load_terms<DT, P>(a, rowp, c, ctx, k, r, L.tab, t);
+        nv = chain_load_terms<DT, P>(a, rowp, et, c, ctx, k, r, L.tab, t);
         if (c == 0) {
             st = head_walk(t, thr, hit);
             if (*hit >= 0) return st;

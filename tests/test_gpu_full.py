@@ -217,3 +217,35 @@ def test_flat_bf16_large_batches(orc, B):
     nb = check(orc, rows, t, k, p, u, ids, o, CAP, f"flat B={B}", probs=(cap == V), threads=16)
     print(f"flat bf16 B={B}: {B} rows bit-exact, boundary draws (|u*P - cum| < 1e-6): {nb}")
     s.close()
+
+
+def test_rows_beyond_the_kept_terms(orc):
+    """A batch of binary32 rows larger than the terms that a handle keeps (64
+    MiB: 64 rows of this vocabulary): the rows before and after the limit, full
+    ones and, interleaved, wide ones (TopK beyond the top-k launch)."""
+    B, K = 68, 3000
+    rows = np.empty((B, V), F32)
+    rng = np.random.default_rng(5)
+    for r in range(B):
+        rows[r] = rng.standard_normal(V, dtype=F32) * 3
+    u = np.floor(rng.random(B) * 2**32) / 2**32
+    t = np.full(B, 0.9, F32)
+    p = np.full(B, 0.97, F32)
+    k = np.zeros(B, np.int32)
+    k[[3, 63, 64, 66]] = K
+    s = native.Sampler(V, max_batch=B, softcap=CAP)
+    d = hip.Buffer.from_array(rows)
+    outs = native.DeviceOutputs(B, K)
+    _, ids = s.sample(d, B, _params(t, k, p), u, outputs=outs.struct)
+    o = outs.read()
+    s.close()
+    look = [0, 1, 3, 62, 63, 64, 65, 66, 67]
+    wide = [r for r in look if k[r]]
+    full = [r for r in look if not k[r]]
+    sub = {n: o[n][full] for n in ("flags", "lsum", "argmax", "count")}
+    check(orc, rows[full], t[full], k[full], p[full], u[full], ids[full], sub, CAP, "kept", threads=8)
+    for r in wide:
+        tok, det, idx, probs = orc.do_sample(rows[r], t[r], k[r], p[r], u[r], softcap=CAP)
+        assert ids[r] == tok and o["count"][r] == det["count"], r
+        assert np.array_equal(o["indices"][r][:K], idx), r
+        assert np.array_equal(o["probs"][r][:K].view(np.uint32), probs.view(np.uint32)), r
