@@ -454,14 +454,15 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
  * wave copies kRowKb blocks of its rows at a time into its own LDS (9 lanes
  * read 144 bytes of a row, seven rows a load; held in registers while the
  * previous stage is summed) and each lane then reads its own row from there.
- * The LDS pitch is an odd number of dwords: no bank conflicts.  Three waves
- * a SIMD (139 VGPRs with 32 vectors).
+ * The LDS pitch is an odd number of dwords: no bank conflicts.  At least three
+ * waves a SIMD (139 VGPRs with 32 vectors; one vector takes 96 and fills the
+ * LDS with 16 waves a compute unit).
  *
  * 262,144 x 2,560: B = 1 652 -> 104 us, B = 8 692 -> 181, B = 32 750 -> 387
  * (one row per thread before, 32 vectors' time for any batch).  B = 1 is
  * bound by the weights' reads, which a stage's ends make 1.7 times their size
- * (a line shared by two stages has left L2 in between: 12 waves a compute
- * unit keep 50 MB in flight; without the sums 95 us).  16 blocks a stage at
+ * (a line shared by two stages has left L2 in between: 4,096 waves keep 70 MB
+ * in flight; without the sums 95 us).  16 blocks a stage at
  * two waves a SIMD take 105, 187 and 387 us, and 100,003 x 1,120 for two
  * vectors 36 us against 30; four waves a SIMD spill at 32 vectors (409 us).
  * ------------------------------------------------------------------ */
