@@ -2,8 +2,9 @@
  * g4s_topk.hip -- the top-k sampling path on gfx950 (rows with 0 < TopK < V).
  *
  * Replaces DoSelectTopKIndices + the top-k branch of DoSample
- * (src/Gemma4.Model.pas:2615-2689, 2765-2826).  One kernel launch per batch,
- * grid = splits x rows, one workgroup per vocabulary chunk:
+ * (src/Gemma4.Model.pas:2615-2689, 2765-2826).  One kernel launch per batch
+ * (bf16: a second one replays the heap of the rows that need it), grid = splits
+ * x rows, one workgroup per vocabulary chunk:
  *
  *  phase 1 (every workgroup)
  *    - 16-byte loads of the chunk into registers as order-preserving keys;
