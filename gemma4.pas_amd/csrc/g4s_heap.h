@@ -20,8 +20,13 @@
  *  - larger K: the nodes are 8-byte LDS entries, a node's children one
  *    16-byte read, and insertions two levels apart run down the heap at the
  *    same time, one per lane: a new one enters every second step, whatever
- *    the depth.  (It makes the reference's comparisons one by one, so it also
- *    takes rows with NaNs, which break the heap's order.)
+ *    the depth.
+ *
+ * A NaN passes every screen and breaks the heap's order: later insertions can
+ * lift it to the root, whatever follows is then accepted, and the root falls.
+ * So from the row's first NaN on (or up to 63 screened elements before it) each
+ * element is compared with the root that it meets, and inserted through the
+ * LDS form, which makes the reference's comparisons one by one.
  *
  * bf16 rows of 262,144 logits, whole calls, before (one lane inserting step by
  * step, tiles of the block's size) and now: K = 64, one row 713 -> 135 us;
@@ -45,7 +50,8 @@ typedef uint64_t HeapPair __attribute__((ext_vector_type(2), may_alias));
 struct HeapCtl {
     int cnt[2][kHeapMaxWaves];  /* entries of each screening wave's segment */
     int stop[2][kHeapMaxWaves]; /* first element that found its segment full, -1: none */
-    float root[2];
+    float root[2];              /* NaN: a NaN was met, */
+    int nan;                    /* at this element or a little behind it */
 };
 
 __device__ __forceinline__ uint64_t heap_pack(float v, int32_t i)
@@ -187,7 +193,6 @@ struct HeapWave {
     {
         const float qv = heap_val(e);
         const int32_t qi = heap_idx(e);
-        if (regs && __builtin_amdgcn_ballot_w64(valid && qv != qv)) spill();
         uint64_t mask = __builtin_amdgcn_ballot_w64(valid && !(qv <= root)); /* :2643-2644 */
         if (regs) {
             while (mask) {
@@ -202,6 +207,23 @@ struct HeapWave {
                 insert_pipe(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(qv), l)),
                             __builtin_amdgcn_readlane(qi, l));
                 mask = (mask & (mask - 1)) & __builtin_amdgcn_ballot_w64(!(qv <= root));
+            }
+        }
+    }
+    /* n elements of the row; the root may fall, so those behind an insertion are
+     * compared again */
+    __device__ __forceinline__ void follow(const uint64_t* e, int n)
+    {
+        if (regs) spill();
+        for (int i = lane; i - lane < n; i += 64) {
+            const uint64_t x = i < n ? e[i] : 0ull;
+            uint64_t mask = __builtin_amdgcn_ballot_w64(i < n && !(heap_val(x) <= root));
+            while (mask) {
+                const int l = (int)__builtin_ctzll(mask);
+                insert_pipe(
+                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(heap_val(x)), l)),
+                    __builtin_amdgcn_readlane(heap_idx(x), l));
+                mask = __builtin_amdgcn_ballot_w64(i < n && lane > l && !(heap_val(x) <= root));
             }
         }
     }
@@ -252,15 +274,22 @@ __device__ __forceinline__ void heap_replay(const char* row, int V, int K, uint6
                 const int c = s < nseg ? ctl.cnt[buf ^ 1][s] : 0;
                 total += __builtin_amdgcn_readfirstlane(c);
             }
+            bool nan = false;
             for (int i = 0; i < total; i += 64) {
                 const int f = i + lane;
                 int at = f;
 #pragma unroll
                 for (int s = 1; s < NP; ++s) at = f >= first[s] ? s * cap + f - first[s] : at;
-                hw.take(f < total ? seg[at] : 0ull, f < total);
+                const uint64_t e = f < total ? seg[at] : 0ull;
+                if (__builtin_amdgcn_ballot_w64(heap_val(e) != heap_val(e))) {
+                    nan = true;
+                    if (lane == 0) ctl.nan = heap_idx(e);
+                    break;
+                }
+                hw.take(e, f < total);
             }
-            if (!more) hw.finish();
-            if (lane == 0) ctl.root[buf] = hw.root;
+            if (!more && !nan) hw.finish();
+            if (lane == 0) ctl.root[buf] = nan ? __builtin_nanf("") : hw.root;
         } else if (more) {
             const int pw = wid - 1;
             uint64_t* seg = q + (buf * NP + pw) * cap;
@@ -315,8 +344,8 @@ __device__ __forceinline__ void heap_replay(const char* row, int V, int K, uint6
             if (lane == 0) ctl.cnt[buf][pw] = total < cap ? total : cap;
         }
         __syncthreads();
-        if (!more) break;
         root = ctl.root[buf];
+        if (!more || root != root) break;
         nseg = 0;
         int64_t next = t0 + (int64_t)NP * n * STEP;
         while (nseg < NP) {
@@ -327,6 +356,18 @@ __device__ __forceinline__ void heap_replay(const char* row, int V, int K, uint6
             }
         }
         pos = next < V ? (int)next : V;
+    }
+    if (__builtin_expect(root != root, 0)) {
+        for (int base = ctl.nan; base < V; base += qn) {
+            const int n = V - base < qn ? V - base : qn;
+            for (int i = threadIdx.x; i < n; i += BLOCK)
+                q[i] = heap_pack(load_elem<DT>(row, base + i), base + i);
+            __syncthreads();
+            if (wid == 0) hw.follow(q, n);
+            __syncthreads();
+        }
+        if (wid == 0) hw.finish();
+        __syncthreads();
     }
 }
 
