@@ -16,27 +16,20 @@ hipError_t lmhead_q4_0_launch(const uint8_t* w, int32_t rows, int32_t cols, cons
 constexpr int kQ4TileRows = 64;
 constexpr int kQ4TileBytes = kQ4TileRows * 4 + kQ4TileRows * 16;
 
-/* Weight j of a block: term (Single(q) * LScale) of CpuMatVecQ4
- * (src/Gemma4.Tensors.pas:586,590) with q = nibble - 8; fma(nibble, s, -8s)
- * is exact and equal to it (both are (nibble - 8) * s, at most 15
- * significant bits).  w: the row's 16 nibble bytes, low nibble of byte j is
- * weight 2j, high nibble weight 2j + 1. */
-__device__ __forceinline__ void q4_dequant32(const uint4 w, float sc, float (&q)[32])
+/* Eight weights of a row, (Single(q) * LScale) of CpuMatVecQ4
+ * (src/Gemma4.Tensors.pas:586,590) with q = nibble - 8: nibble t of `w` is
+ * weight t.  A nibble with its top bit flipped is q in two's complement, which
+ * v_cvt_off_f32_i4 gives as a sixteenth from any byte's low half.  s16 = 16 s.
+ * One product as in the reference, so infinite scales come out the same. */
+__device__ __forceinline__ void q4_dequant8(uint32_t w, float s16, float (&q)[8])
 {
-    const float m8 = -8.0f * sc;
-    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+    const uint32_t lo = w ^ 0x88888888u;
+    uint32_t hi; /* opaque, or its bytes are extracted from lo one by one */
+    asm("v_lshrrev_b32 %0, 4, %1" : "=v"(hi) : "v"(lo));
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        /* the nibble masks stay opaque so that each nibble converts with one
-         * v_cvt_f32_ubyteN (instead of a field extract and a convert) */
-        uint32_t lo, hi;
-        asm("v_and_b32 %0, 0x0f0f0f0f, %1" : "=v"(lo) : "v"(ws[d]));
-        asm("v_and_b32 %0, 0x0f0f0f0f, %1" : "=v"(hi) : "v"(ws[d] >> 4));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            q[8 * d + 2 * i] = __builtin_fmaf((float)((lo >> (8 * i)) & 0xFFu), sc, m8);
-            q[8 * d + 2 * i + 1] = __builtin_fmaf((float)((hi >> (8 * i)) & 0xFFu), sc, m8);
-        }
+    for (int i = 0; i < 4; ++i) {
+        q[2 * i] = __builtin_amdgcn_cvt_off_f32_i4((int)((lo >> (8 * i)) & 0xFFu)) * s16;
+        q[2 * i + 1] = __builtin_amdgcn_cvt_off_f32_i4((int)((hi >> (8 * i)) & 0xFFu)) * s16;
     }
 }
 

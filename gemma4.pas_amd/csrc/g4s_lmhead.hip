@@ -14,7 +14,10 @@
  * of a midpoint, which happens only for 0 < |S| <= 2^-64 |q*s*x| with q*s*x
  * itself a binary32 midpoint -- never for this workload (|S| is then at
  * least 2^-60 unless it is 0).  So the kernel is one fma per term, in the
- * reference's order.
+ * reference's order.  A weight of zero counts as +0 where the reference may
+ * have -0: that shows only in a running sum of -0, as the sign of a zero logit,
+ * and such a sum takes a product that underflows to zero (a scale is 0 or at
+ * least 2^-14, so a hidden value below 2^-135).
  *
  * Every wave owns 64 weight rows (lane = row) and some hidden vectors: one
  * accumulator form per number of vectors, over either layout of the weights.
@@ -96,7 +99,8 @@ typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(1)));
 /* Eight weights of a row: nibble t of `w` is weight t.  A byte 0..15 read as
  * fp8 (e4m3) is n * 2^-9 (its denormals and first binade), so one
  * v_cvt_pk_f32_fp8 gives two nibbles, and fma(n * 2^-9, 512 s, -8 s) is
- * (n - 8) s exactly (at most 15 significant bits).  s512 = 512 s, m8 = -8 s. */
+ * (n - 8) s exactly (at most 15 significant bits), a zero being +0.  An infinite
+ * s gives NaN (sum_infinite).  s512 = 512 s, m8 = -8 s. */
 __device__ __forceinline__ void dequant8(uint32_t w, float s512, float m8, float (&q)[8])
 {
     const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
@@ -400,6 +404,44 @@ struct FewAcc {
     }
 };
 
+/* smax: the largest scale of a lane's row.  (Of fmaxf the compiler makes one
+ * v_max3_f32 for two blocks and waits for the second block's loads before the
+ * first is summed: 76.5 us instead of 74.9 for one vector.) */
+__device__ __forceinline__ void max_scale(float& smax, float s)
+{
+    asm("v_max_f32 %0, %0, |%1|" : "+v"(smax) : "v"(s));
+}
+
+/* The sums of the rows with an infinite scale, of which dequant8 makes NaN,
+ * taken again with the reference's product.  Waves without such a row end at
+ * the test (262,144 x 2,560: 74.9 us for one vector, 368 for 32; with
+ * q4_dequant8 for every sum 76.8 and 371.6).  block(k, s, w): the lane's block
+ * k; rows that are not live have sums that nobody reads. */
+template <int VECS, typename Block, typename Put>
+__device__ __forceinline__ void sum_infinite(float smax, bool live, const float* h, int32_t cols,
+                                             int32_t nblk, int32_t b0, int32_t batch, Block block,
+                                             Put put)
+{
+    if (__builtin_expect(__ballot(live && smax == __builtin_inff()) == 0, 1)) return;
+    for (int32_t i = 0; i < VECS && b0 + i < batch; ++i) {
+        const float* x = h + (int64_t)(b0 + i) * cols;
+        float S = 0.0f;
+        for (int32_t k = 0; k < nblk; ++k, x += 32) {
+            float s;
+            uint32_t w[4];
+            block(k, s, w);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                float q[8];
+                q4_dequant8(w[d], 16.0f * s, q);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) S = __builtin_fmaf(q[j], x[8 * d + j], S);
+            }
+        }
+        put(S, i);
+    }
+}
+
 template <typename Acc, int DEPTH>
 __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
     const uint8_t* __restrict__ tiles, int32_t rows, int32_t nblk, const float* __restrict__ h,
@@ -413,7 +455,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
     const uint8_t* tp = tiles + (int64_t)g * nblk * kQ4TileBytes;
     Acc acc;
     acc.init(h, cols, b0, batch, lane);
-    float sc[DEPTH];
+    float sc[DEPTH], smax = 0.0f;
     uint4 w[DEPTH];
     typename Acc::X x[DEPTH];
     const auto fetch = [&](int d, int32_t k) {
@@ -431,6 +473,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
     for (; k + DEPTH <= nblk; k += DEPTH) {
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
+            max_scale(smax, sc[d]);
             acc.mac(w[d], sc[d], x[d]);
             const int32_t kn = k + d + DEPTH;
             fetch(d, kn < nblk ? kn : nblk - 1);
@@ -439,12 +482,24 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
         }
     }
 #pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d)
-        if (k + d < nblk) acc.mac(w[d], sc[d], x[d]);
+    for (int d = 0; d < DEPTH - 1; ++d) {
+        if (k + d < nblk) {
+            max_scale(smax, sc[d]);
+            acc.mac(w[d], sc[d], x[d]);
+        }
+    }
     const int32_t r = g * kQ4TileRows + lane;
-    acc.emit([&](float v, int i) {
+    const auto put = [&](float v, int i) {
         if (b0 + i < batch) put_logit(v, b0 + i, r, rows, lane, g, ngroups, out, stride, gsum);
-    });
+    };
+    acc.emit(put);
+    const auto block = [&](int32_t kb, float& s, uint32_t (&q)[4]) {
+        const uint8_t* t = tp + (uint32_t)kb * (uint32_t)kQ4TileBytes;
+        s = reinterpret_cast<const float*>(t)[lane];
+        const uint4 n = reinterpret_cast<const uint4*>(t + kQ4TileRows * 4)[lane];
+        q[0] = n.x, q[1] = n.y, q[2] = n.z, q[3] = n.w;
+    };
+    sum_infinite<Acc::kVecs>(smax, r < rows, h, cols, nblk, b0, batch, block, put);
 }
 
 /* ------------------------------------------------------------------
@@ -537,6 +592,7 @@ __global__ __launch_bounds__(64, 3) void lmhead_rows_kernel(
     Acc acc;
     acc.init(h, cols, b0, batch, lane);
     typename Acc::X x[DEPTH];
+    float smax = 0.0f;
     if (!edge(0)) {
 #pragma unroll
         for (int j = 0; j < kRowLoads; ++j) fetch(j, 0);
@@ -588,7 +644,9 @@ __global__ __launch_bounds__(64, 3) void lmhead_rows_kernel(
                 half = e[4] >> 16;
                 w = make_uint4(e[5], e[6], e[7], e[8]);
             }
-            acc.mac(w, f16_to_f32_fast(half), x[i % DEPTH]);
+            const float sc = f16_to_f32_fast(half);
+            max_scale(smax, sc);
+            acc.mac(w, sc, x[i % DEPTH]);
             const int32_t kn = k + DEPTH;
             acc.load(x[i % DEPTH], kn < nblk ? kn : nblk - 1);
             __builtin_amdgcn_sched_barrier(0);
@@ -596,9 +654,18 @@ __global__ __launch_bounds__(64, 3) void lmhead_rows_kernel(
         __builtin_amdgcn_wave_barrier(); /* the next stage is written after these reads */
     }
     const int32_t r = r0 + lane;
-    acc.emit([&](float v, int i) {
-        if (b0 + i < batch && r >= own && r < rows) out[(int64_t)(b0 + i) * stride + r] = v;
-    });
+    const bool live = r >= own && r < rows;
+    const auto write = [&](float v, int i) {
+        if (b0 + i < batch && live) out[(int64_t)(b0 + i) * stride + r] = v;
+    };
+    acc.emit(write);
+    const auto block = [&](int32_t kb, float& s, uint32_t (&q)[4]) {
+        const uint8_t* b = wt + (int64_t)(live ? r : own) * pitch + kb * 18;
+        s = f16_to_f32_ref((uint32_t)b[0] | ((uint32_t)b[1] << 8));
+        const uint4u n = *reinterpret_cast<const uint4u*>(b + 2);
+        q[0] = n.x, q[1] = n.y, q[2] = n.z, q[3] = n.w;
+    };
+    sum_infinite<Acc::kVecs>(smax, live, h, cols, nblk, b0, batch, block, write);
 }
 
 /* DoEmbeddingLookup for a Q4_0 table (src/Gemma4.Model.pas:2047-2080):

@@ -1352,17 +1352,14 @@ __global__ __launch_bounds__(kGlThreads) void group_logits_kernel(TopkArgs a)
         for (int q = 0; q < kGlItems; ++q) {
             const int it = p + q * kGlProd;
             const float sc = rsc[SLOT][q];
-            const float m8 = -8.0f * sc;
             const uint32_t ws[2] = {rq0[SLOT][q], rq1[SLOT][q]};
             float w[16];
 #pragma unroll
             for (int d = 0; d < 2; ++d) {
-                const uint32_t lo = ws[d] & 0x0F0F0F0Fu, hi = (ws[d] >> 4) & 0x0F0F0F0Fu;
+                float w8[8];
+                q4_dequant8(ws[d], 16.0f * sc, w8);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    w[8 * d + 2 * i] = __builtin_fmaf((float)((lo >> (8 * i)) & 0xFFu), sc, m8);
-                    w[8 * d + 2 * i + 1] = __builtin_fmaf((float)((hi >> (8 * i)) & 0xFFu), sc, m8);
-                }
+                for (int i = 0; i < 8; ++i) w[8 * d + i] = w8[i];
             }
             float4* dst = reinterpret_cast<float4*>(
                 &s_w[buf][it >> 7][((it >> 1) & 63) * kGlStride + (it & 1) * 16]);

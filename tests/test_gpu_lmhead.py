@@ -123,6 +123,42 @@ def test_lmhead_scale_edge_cases(orc):
     s.close()
 
 
+@pytest.mark.parametrize("batch", [1, 2, 3, 9, 13, 17, 25, 30])
+@pytest.mark.parametrize("rows", [64, 64 * 1025 + 5])  # a vector a wave and all of them
+@pytest.mark.parametrize("layout", ["rows", "tiled"])
+def test_lmhead_infinite_scales(orc, layout, rows, batch):
+    """Infinite and NaN scales: (nibble - 8) * s is an infinity, NaN for nibble
+    8; the rows beside them keep their sums."""
+    cols = 3 * 32
+    w = wl.host_q4_weights(83, rows, cols).reshape(rows, 3, 18)
+    rng = np.random.default_rng(6)
+    w[:, 1, 2:] = rng.choice([0x99, 0xA9, 0xFB], (rows, 16))                  # 1..7: one sign
+    w[8::16, 1, 2:] = rng.choice([0x91, 0x28, 0xF0], (len(w[8::16]), 16))     # mixed signs, zeros
+    for i, v in enumerate([0x7C00, 0xFC00, 0x7E00, 0x7BFF]):
+        w[i::8, 1, 0], w[i::8, 1, 1] = v & 0xFF, v >> 8
+    hidden = np.abs(rng.normal(0, 1, (batch, cols))).astype(F32)
+    hidden[1::3] *= -1
+    s = native.Sampler(V, max_batch=1, softcap=30.0)
+    if layout == "rows":
+        got = _lmhead(s, w.reshape(-1), rows, cols, hidden)
+    else:
+        src = hip.Buffer.from_array(w.reshape(-1))
+        tiles = hip.Buffer(native.q4_0_device_bytes(rows, cols, native.Q4_LAYOUT_TILED64))
+        native.q4_0_repack(src, rows, cols, tiles)
+        dh = hip.Buffer.from_array(hidden)
+        dl = hip.Buffer(4 * batch * rows)
+        s.lmhead_q4_0_tiled(tiles, rows, cols, dh, batch, dl, rows)
+        hip.synchronize()
+        got = dl.download(F32).reshape(batch, rows)
+    s.close()
+    want = orc.matvec_q4_batch(w.reshape(-1), hidden, rows, cols, threads=8)
+    nan = np.isnan(want)
+    assert nan.any() and np.isposinf(want).any() and (batch < 2 or np.isneginf(want).any())
+    assert np.array_equal(np.isnan(got), nan)
+    bad = got.view(np.uint32)[~nan] != want.view(np.uint32)[~nan]
+    assert not bad.any(), f"{bad.sum()} logits differ"
+
+
 def test_lmhead_hand_built_blocks():
     """Hand-built Q4_0 blocks with written-out expected logits: byte j holds
     element 2j in its low nibble and 2j+1 in its high nibble (Tensors.pas:

@@ -413,3 +413,26 @@ def test_fused_no_logits_rejects_full_rows(orc):
         rc, _ = s.lmhead_sample_q4_0(d_tile, cols, dh, 2, None, params, [0.5, 0.5], check=False)
         assert rc == native.G4S_ERR_INVALID_ARGUMENT, (kk, rc, s.last_error())
     s.close()
+
+
+def test_fused_no_logits_infinite_scales(orc):
+    """Rows whose infinite scale makes their logit an infinity, several in one
+    group: the head's summaries and the recomputed groups agree on them."""
+    vocab, cols, B = 9000, 64, 4
+    w = wl.host_q4_weights(141, vocab, cols).reshape(vocab, cols // 32, 18)
+    for r, s16 in [(10, 0x7C00), (11, 0x7C00), (40, 0xFC00), (700, 0x7C00), (703, 0xFC00)]:
+        w[r, 0, 0], w[r, 0, 1] = s16 & 0xFF, s16 >> 8
+        w[r, 0, 2:] = 0xA9
+    w = w.reshape(-1)
+    d_tile = hip.Buffer(native.q4_0_device_bytes(vocab, cols, native.Q4_LAYOUT_TILED64))
+    d_rows = hip.Buffer.from_array(w)
+    native.q4_0_repack(d_rows, vocab, cols, d_tile)
+    hip.synchronize()
+    hidden = np.abs(wl.host_hidden(142, B, cols))
+    want = orc.matvec_q4_batch(w, hidden, vocab, cols)
+    assert np.all(np.isposinf(want).sum(axis=1) == 3) and not np.isnan(want).any()
+    k = np.array([2, 5, 40, 300], np.int32)
+    s = native.Sampler(vocab, max_batch=B, softcap=30.0)
+    _no_logits_check(orc, s, d_tile, w, hidden, np.full(B, 0.7, F32), k, np.full(B, 0.95, F32),
+                     wl.host_row_u(143, 0, B), "inf", capacity=300)
+    s.close()
