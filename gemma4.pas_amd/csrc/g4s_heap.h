@@ -24,9 +24,9 @@
  *
  * A NaN passes every screen and breaks the heap's order: later insertions can
  * lift it to the root, whatever follows is then accepted, and the root falls.
- * So from the row's first NaN on (or up to 63 screened elements before it) each
- * element is compared with the root that it meets, and inserted through the
- * LDS form, which makes the reference's comparisons one by one.
+ * So from the stretch that holds the row's first NaN on each element is compared
+ * with the root that it meets, and inserted through the LDS form, which makes
+ * the reference's comparisons one by one.
  *
  * bf16 rows of 262,144 logits, whole calls, before (one lane inserting step by
  * step, tiles of the block's size) and now: K = 64, one row 713 -> 135 us;
@@ -43,15 +43,15 @@ namespace g4s {
 
 constexpr int kHeapExtra = 4;   /* entries beyond K: node 0 and the children past the last node */
 constexpr int kHeapMaxWaves = 16;
+constexpr int kHeapNan = 1 << 20; /* above any number of entries */
 
 /* two entries; may_alias: the same memory is written as single entries */
 typedef uint64_t HeapPair __attribute__((ext_vector_type(2), may_alias));
 
 struct HeapCtl {
-    int cnt[2][kHeapMaxWaves];  /* entries of each screening wave's segment */
+    int cnt[2][kHeapMaxWaves];  /* entries of each screening wave's segment, kHeapNan if NaNs passed */
     int stop[2][kHeapMaxWaves]; /* first element that found its segment full, -1: none */
-    float root[2];              /* NaN: a NaN was met, */
-    int nan;                    /* at this element or a little behind it */
+    float root[2];              /* NaN: there is one in the stretch */
 };
 
 __device__ __forceinline__ uint64_t heap_pack(float v, int32_t i)
@@ -253,7 +253,7 @@ __device__ __forceinline__ void heap_replay(const char* row, int V, int K, uint6
     __syncthreads(); /* the areas are free */
     if (wid == 0) hw.init(heap, K, lane);
     float root = -1e30f;
-    int pos = 0, nseg = 0;
+    int pos = 0, from = 0, nseg = 0;
     for (int ph = 0;; ++ph) {
         const int buf = ph & 1;
         const bool more = pos < V;
@@ -267,26 +267,23 @@ __device__ __forceinline__ void heap_replay(const char* row, int V, int K, uint6
         if (wid == 0) {
             /* the segments one after another, 64 elements at a time */
             const uint64_t* seg = q + (buf ^ 1) * NP * cap;
-            int first[NP], total = 0; /* a segment's first element in that order */
+            int first[NP], total = 0, nan = 0; /* a segment's first element in that order */
 #pragma unroll
             for (int s = 0; s < NP; ++s) {
                 first[s] = total;
-                const int c = s < nseg ? ctl.cnt[buf ^ 1][s] : 0;
-                total += __builtin_amdgcn_readfirstlane(c);
+                const int c =
+                    __builtin_amdgcn_readfirstlane(s < nseg ? ctl.cnt[buf ^ 1][s] : 0);
+                nan |= c;
+                total += c;
             }
-            bool nan = false;
+            nan &= kHeapNan;
+            if (nan) total = 0;
             for (int i = 0; i < total; i += 64) {
                 const int f = i + lane;
                 int at = f;
 #pragma unroll
                 for (int s = 1; s < NP; ++s) at = f >= first[s] ? s * cap + f - first[s] : at;
-                const uint64_t e = f < total ? seg[at] : 0ull;
-                if (__builtin_amdgcn_ballot_w64(heap_val(e) != heap_val(e))) {
-                    nan = true;
-                    if (lane == 0) ctl.nan = heap_idx(e);
-                    break;
-                }
-                hw.take(e, f < total);
+                hw.take(f < total ? seg[at] : 0ull, f < total);
             }
             if (!more && !nan) hw.finish();
             if (lane == 0) ctl.root[buf] = nan ? __builtin_nanf("") : hw.root;
@@ -295,6 +292,7 @@ __device__ __forceinline__ void heap_replay(const char* row, int V, int K, uint6
             uint64_t* seg = q + (buf * NP + pw) * cap;
             const int64_t w0 = t0 + (int64_t)pw * n * STEP + lane * VW;
             int total = 0;
+            bool nan = false;
             if (lane == 0) ctl.stop[buf][pw] = -1;
             const auto screen = [&](const float(&x)[VW], int64_t e0) __attribute__((always_inline)) {
                 uint32_t in = 0;
@@ -307,6 +305,7 @@ __device__ __forceinline__ void heap_replay(const char* row, int V, int K, uint6
 #pragma unroll
                 for (int i = 0; i < VW; ++i) {
                     if ((in >> i) & 1u) {
+                        nan |= !(x[i] > root);
                         if (at < cap)
                             seg[at] = heap_pack(x[i], (int32_t)(e0 + i));
                         else if (at == cap)
@@ -341,7 +340,8 @@ __device__ __forceinline__ void heap_replay(const char* row, int V, int K, uint6
                     }
                 }
             }
-            if (lane == 0) ctl.cnt[buf][pw] = total < cap ? total : cap;
+            const int bad = __builtin_amdgcn_ballot_w64(nan) ? kHeapNan : 0;
+            if (lane == 0) ctl.cnt[buf][pw] = (total < cap ? total : cap) | bad;
         }
         __syncthreads();
         root = ctl.root[buf];
@@ -355,10 +355,11 @@ __device__ __forceinline__ void heap_replay(const char* row, int V, int K, uint6
                 break;
             }
         }
+        from = pos; /* what the next phase inserts begins here */
         pos = next < V ? (int)next : V;
     }
     if (__builtin_expect(root != root, 0)) {
-        for (int base = ctl.nan; base < V; base += qn) {
+        for (int base = from; base < V; base += qn) {
             const int n = V - base < qn ? V - base : qn;
             for (int i = threadIdx.x; i < n; i += BLOCK)
                 q[i] = heap_pack(load_elem<DT>(row, base + i), base + i);
