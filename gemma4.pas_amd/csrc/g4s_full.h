@@ -133,6 +133,7 @@ struct BfStage {
 static_assert(sizeof(BfStage) % 16 == 0, "BfStage copies in 16-byte units");
 
 struct FullWorkspace {
+    void* base = nullptr;        /* the allocation that holds all of them */
     FullRow* rows = nullptr;     /* [max_batch] */
     FullChunk* chunks = nullptr; /* [max_batch][cstride] */
     ss::PMap* lmap = nullptr;    /* [max_batch][cstride] chunk's terms in beta_l */

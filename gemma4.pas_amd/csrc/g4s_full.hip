@@ -58,6 +58,7 @@
  * sum is the reference's left-to-right binary32 sum, bit for bit.
  */
 #include <climits>
+#include <type_traits>
 
 #include "g4s_fullcore.h"
 #include "g4s_heap.h"
@@ -1090,59 +1091,62 @@ bool full_supported(int32_t vocab)
  * rows takes; a hundred such rows 347 -> 321 us, 64 rows 253 -> 160). */
 constexpr size_t kEtermBytes = (size_t)64 << 20;
 
+/* One allocation for everything: g4s_create pays for each (256 rows of 262,144
+ * with nineteen 395-406 us, with one 180; 4 rows 121 and 101-111, 32 rows 160
+ * and 124-148). */
 hipError_t full_alloc(FullWorkspace& ws, int32_t vocab, int32_t max_batch)
 {
     const size_t mb = (size_t)max_batch;
     ws.bits_stride = (vocab + 31) / 32;
     ws.cstride = (vocab + kFullChunk - 1) / kFullChunk;
     const size_t nc = mb * (size_t)ws.cstride;
-    hipError_t e = hipMalloc((void**)&ws.rows, mb * sizeof(FullRow));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.chunks, nc * sizeof(FullChunk));
-    /* the two maps, binades and tables share an allocation each */
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.lmap, 2 * nc * sizeof(PMap));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.beta_l, 2 * nc * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.etab, 2 * mb * kFullTab * sizeof(float));
-    if (e == hipSuccess) {
-        ws.cmap = ws.lmap + nc;
-        ws.beta_c = ws.beta_l + nc;
-        ws.ptab = ws.etab + mb * kFullTab;
+    /* the layout: sizes are counted with no base, then the pointers set */
+    const auto lay = [&](char* base) {
+        size_t at = 0;
+        const auto put = [&](auto*& p, size_t n) {
+            if (base) p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + at);
+            at += (n * sizeof(*p) + 255) & ~(size_t)255;
+        };
+        put(ws.rows, mb);
+        put(ws.chunks, nc);
+        put(ws.lmap, nc);
+        put(ws.cmap, nc);
+        put(ws.beta_l, nc);
+        put(ws.beta_c, nc);
+        put(ws.etab, mb * kFullTab);
+        put(ws.ptab, mb * kFullTab);
+        put(ws.tmask, mb * 2);
+        put(ws.sel, mb);
+        put(ws.hist, mb * kWideBins);
+        put(ws.ties, mb * kSelMaxChunks);
+        put(ws.bits, mb * (size_t)ws.bits_stride);
+        put(ws.heap, (size_t)vocab + kHeapExtra);
+        put(ws.ytab, (size_t)65536);
+        put(ws.fbrow, mb);
+        put(ws.etab8, mb * kBfTab);
+        put(ws.ptab8, mb * kBfTab);
+        put(ws.stage, mb * kBfStage);
+        put(ws.cpost, nc);
+        put(ws.head, mb * kFullChunk);
+        put(ws.eterm, (size_t)ws.erows * (size_t)ws.cstride * kFullChunk);
+        return at;
+    };
+    const size_t rows = kEtermBytes / ((size_t)ws.cstride * kFullChunk * sizeof(float));
+    ws.erows = (int32_t)(rows < mb ? rows : mb);
+    hipError_t e = hipMalloc(&ws.base, lay(nullptr));
+    if (e != hipSuccess && ws.erows) {
+        /* without the kept terms the passes evaluate them again */
+        (void)hipGetLastError();
+        ws.erows = 0;
+        e = hipMalloc(&ws.base, lay(nullptr));
     }
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.tmask, mb * 2 * sizeof(uint64_t));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.sel, mb * sizeof(WideSel));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.hist, mb * kWideBins * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.ties, mb * kSelMaxChunks * sizeof(TieRec));
-    if (e == hipSuccess)
-        e = hipMalloc((void**)&ws.bits, mb * (size_t)ws.bits_stride * sizeof(uint32_t));
-    if (e == hipSuccess)
-        e = hipMalloc((void**)&ws.heap, ((size_t)vocab + kHeapExtra) * sizeof(uint64_t));
-    if (e == hipSuccess) {
-        /* without it (or beyond it) the passes evaluate the terms again */
-        const size_t per = (size_t)ws.cstride * kFullChunk * sizeof(float);
-        const size_t rows = kEtermBytes / per;
-        ws.erows = (int32_t)(rows < mb ? rows : mb);
-        if (ws.erows && hipMalloc((void**)&ws.eterm, ws.erows * per) != hipSuccess) {
-            (void)hipGetLastError();
-            ws.eterm = nullptr;
-            ws.erows = 0;
-        }
-    }
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.ytab, (size_t)65536 * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.fbrow, mb * sizeof(FbRow));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.etab8, mb * kBfTab * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.ptab8, mb * kBfTab * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.stage, mb * kBfStage * sizeof(BfStage));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.cpost, nc * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void**)&ws.head, mb * kFullChunk * sizeof(float));
+    if (e == hipSuccess) (void)lay(static_cast<char*>(ws.base));
     return e;
 }
 
 void full_free(FullWorkspace& ws)
 {
-    void* ptrs[] = {ws.rows, ws.chunks, ws.lmap, ws.beta_l, ws.etab, ws.tmask, ws.sel, ws.hist,
-                    ws.ties, ws.bits, ws.heap, ws.eterm, ws.ytab, ws.fbrow,
-                    ws.etab8, ws.ptab8, ws.stage, ws.cpost, ws.head};
-    for (void* p : ptrs)
-        if (p) (void)hipFree(p);
+    if (ws.base) (void)hipFree(ws.base);
     ws = FullWorkspace{};
 }
 
