@@ -202,6 +202,11 @@ struct HeapWave {
                 mask = (mask & (mask - 1)) & __builtin_amdgcn_ballot_w64(!(qv <= root));
             }
         } else {
+            /* the loop's place in the 32-byte windows of instruction fetch: K =
+             * 1,100 takes 1,836 us (four rows of 262,144) where it ends up with five
+             * s_nop, 1,849 with two or three, 1,862 with four, 1,910 with six and
+             * 1,938 with none or eight; without this it moves with any change */
+            asm volatile(".p2align 6\ns_nop 0\ns_nop 0\ns_nop 0\ns_nop 0\ns_nop 0");
             while (mask) {
                 const int l = (int)__builtin_ctzll(mask);
                 insert_pipe(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(qv), l)),
