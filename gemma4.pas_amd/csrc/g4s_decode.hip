@@ -112,7 +112,8 @@ __device__ __forceinline__ void load4(const char* row, int64_t e0, int64_t limit
  * tiles of 1024 elements screened against the current root (an element at
  * or below it would be rejected by every later root too), the screened ones
  * inserted in index order by one lane with the reference's comparisons; the
- * next tile is loaded while one is screened.  On return hv[0..K) / hi[0..K)
+ * next tile is loaded while one is screened.  Exact for rows without NaNs:
+ * behind a NaN the root can fall inside a tile.  On return hv[0..K) / hi[0..K)
  * hold the heap (hi = -1 where the row had fewer than K logits above -1e30). */
 template <typename SH>
 __device__ void replay_heap(const char* row, int V, int K, SH& sh, float* hv, int32_t* hi)

@@ -693,8 +693,10 @@ __global__ __launch_bounds__(kFullBlock) void full_lsum_kernel(FullArgs a)
  * operations a term: at 16 terms a lane one row is 256 waves of 16 chains each
  * (16.7 us, here 7.8; 24 rows of 100,003 22.8 us, here 16.7).  Kept, the terms
  * are not evaluated again by the draw's pass (18.9 -> 5.1 us, 37.3 -> 8.5) and
- * by the staged chunks of the two chains (38.4 and 41.2 -> 25 us each).  The
- * 100th row of a batch is beyond them: such rows take full_lsum_kernel. */
+ * by the staged chunks of the two chains (38.4 and 41.2 -> 25 us each).  Rows
+ * from a.ws.erows on (kEtermBytes over a row's terms: 64 rows of 262,144, 167 of
+ * 100,003; none where they could not be allocated) take full_lsum_kernel and
+ * full_cdf_kernel. */
 static_assert(kFullBlock * 4 == kFullChunk, "four terms per thread");
 __global__ __launch_bounds__(kFullBlock) void full_lsum_store_kernel(FullArgs a)
 {

@@ -2,15 +2,18 @@
  * g4s_heap.h -- exact replay of the reference's min-heap pass
  * (DoSelectTopKIndices, src/Gemma4.Model.pas:2632-2664) over a whole row, for
  * rows whose K-th value is tied in a way the heap's layout decides (bf16
- * logits: nearly every row).  Used by the top-k kernels (g4s_decode.hip,
- * g4s_topk.hip) and the wide select (g4s_full.hip).
+ * logits: nearly every row).  Used by the launch that follows a bf16 top-k
+ * select (g4s_topk.hip) and by the wide select (g4s_full.hip).
  *
  * About K (1 + ln(V / K)) elements enter the heap, each after the one before,
- * so the replay is bound by the latency of one insertion.  The heap's root
- * only rises, so screening against an older root keeps a superset: waves 1..
- * screen the next stretch of the row into LDS (as long as half of what
- * precedes it, read 16 bytes a lane, several loads in flight) while wave 0
- * inserts from the stretch before.  Wave 0 inserts in one of two ways:
+ * so the replay is bound by the latency of one insertion.  Without NaNs the
+ * heap's root only rises, so screening against an older root keeps a superset:
+ * waves 1.. screen the next stretch of the row into LDS (as long as what
+ * precedes it, less where the segments would overflow; read 16 bytes a lane,
+ * several loads in flight) while wave 0 inserts from the stretch before.  The
+ * first stretches admit one segment each (every element passes the first root),
+ * so 100,003 elements with K = 40 take nine phases.  Wave 0 inserts in one of
+ * two ways:
  *
  *  - K <= 64: node j of the heap lives in lane j (node 64 in lane 0).  The
  *    smaller child of every node is known before the value is: its ballot

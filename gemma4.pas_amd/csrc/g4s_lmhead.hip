@@ -161,7 +161,7 @@ __device__ __forceinline__ void mac32(f32x4 (&S)[NG], const uint4 w, float sc, c
  * scale and 16 nibble bytes from the tile (256 + 1024 contiguous bytes per
  * wave) and two columns of its vectors (L1/L2 hits), kept DEPTH blocks ahead
  * in registers.  262,144 x 2,560 (a plain read of the 419 MB of tiles takes
- * 69-73 us): B = 1 645 -> 75 us, B = 8 152 us, B = 32 649 -> 361 us.
+ * 69-73 us): B = 1 636 -> 74 us, B = 8 639 -> 147, B = 32 642 -> 361-368.
  * ------------------------------------------------------------------ */
 
 constexpr int kTileWaves = 4; /* waves (64-row groups) per workgroup */
@@ -270,7 +270,7 @@ __device__ __forceinline__ void mac8x32(f32x32& S, const float (&q)[8], const fl
 /* 32 vectors per wave on v_mfma_f32_32x32x1_2b: also one product per output,
  * the weights' two blocks being rows 0-31 and 32-63 and CBSZ = 1 handing
  * either half of the A register to both.  It reads eight times fewer operands
- * per fma than the 4x4 form (262,144 x 2,560 x 32: 361 against 391 us). */
+ * per fma than the 4x4 form (262,144 x 2,560 x 32: 364 against 396 us). */
 struct WideAcc {
     static constexpr int kVecs = 32;
     struct X {
@@ -509,11 +509,12 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void lmhead_tiled_kernel(
  * wave copies kRowKb blocks of its rows at a time into its own LDS (9 lanes
  * read 144 bytes of a row, seven rows a load; held in registers while the
  * previous stage is summed) and each lane then reads its own row from there.
- * The LDS pitch is an odd number of dwords: no bank conflicts.  At least three
- * waves a SIMD (139 VGPRs with 32 vectors; one vector takes 96 and fills the
- * LDS with 16 waves a compute unit).
+ * The LDS pitch is an odd number of dwords, so the reads have no bank conflicts
+ * (the copies, 16 bytes a lane over rows of that pitch, have some: 3.1 M cycles
+ * over 256 compute units).  At least three waves a SIMD (141 VGPRs with 32
+ * vectors; one vector takes 95 and fills the LDS with 16 waves a compute unit).
  *
- * 262,144 x 2,560: B = 1 652 -> 104 us, B = 8 692 -> 181, B = 32 750 -> 387
+ * 262,144 x 2,560: B = 1 652 -> 102 us, B = 8 667 -> 177, B = 32 740 -> 380-390
  * (one row per thread before, 32 vectors' time for any batch).  B = 1 is
  * bound by the weights' reads, which a stage's ends make 1.7 times their size
  * (a line shared by two stages has left L2 in between: 4,096 waves keep 70 MB
@@ -718,11 +719,12 @@ hipError_t q4_tile_launch(const uint8_t* src, int32_t rows, int32_t nblk, uint8_
  *  - every (row group, vector) pair its own wave while that leaves at most
  *    one wave per SIMD, and up to two vectors otherwise: the plain fma kernel
  *    (2,560 columns: 20 us for 8,000 rows x 8 against 31 us with four vectors
- *    a wave; 262,144 rows: 74 us for one vector against 105, 81 for two);
+ *    a wave; 262,144 rows: 74 us for one vector against 105, 85-91 for two);
  *  - else 4 * NG vectors a wave on the matrix cores, NG as large as needed
  *    (up to 8) to leave at most one wave per SIMD (32,768 rows x 32: NG = 4
- *    64 us, NG = 2 75, NG = 8 102; 262,144 rows x 32: NG = 8 391 us, NG = 4
- *    416), and the 32-vector form where a wave takes 29 to 32.
+ *    66 us, NG = 2 75, NG = 8 105; 262,144 rows x 32: NG = 8 396 us, NG = 4
+ *    460), and the 32-vector form where a wave takes 29 to 32 (364 us; at 28 it
+ *    takes 359 against 354 with NG = 7).
  * launch(accumulator, prefetch depth, slices of the batch) starts the kernel. */
 constexpr int32_t kLmSimds = 1024;
 

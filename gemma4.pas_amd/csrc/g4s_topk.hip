@@ -91,9 +91,10 @@ struct TopkShared {
 
 /* Exact replay of the reference's min-heap pass (Model.pas:2632-2664) over a
  * whole row, for binary32 rows whose K-th value is tied in a way the heap
- * layout decides (bf16 rows: topk_replay_kernel).  Elements are screened in tiles against the current root; the
- * screened ones (in index order) are inserted by one lane.  On return
- * hv[0..K) / hi[0..K) hold the heap. */
+ * layout decides (bf16 rows: topk_replay_kernel).  Elements are screened in
+ * tiles against the current root; the screened ones (in index order) are
+ * inserted by one lane.  Exact for rows without NaNs: behind a NaN the root can
+ * fall inside a tile.  On return hv[0..K) / hi[0..K) hold the heap. */
 template <int BLOCK, typename SH>
 __device__ void heap_replay_f32(const char* row, int vocab, int K, SH& sh, float* hv, int32_t* hi)
 {
@@ -991,8 +992,11 @@ constexpr int kReplayQueue = 4096;
 
 /* The rows that the launch before left to a replay of the heap (bf16 logits:
  * nearly every row, ties being ordinary there): one workgroup per row, the
- * other rows' end at once (a synchronous call without ties takes 25.6 us with
- * and without this launch).  Inlined in the kernels that find the tie, the
+ * other rows' end at once.  Where no row is tied the launch costs a
+ * stream-ordered call 1.5 to 2 us (one row of 262,144, K = 8: 10.3 -> 12.3; 64
+ * rows 81.7 -> 83.3) and a synchronous one nothing (22.3 us, the host has its
+ * completion word by then); where one is, it saves hundreds (five rows of
+ * 100,003, K = 40: 400 -> 83).  Inlined in the kernels that find the tie, the
  * replay takes registers from every row (64 mixed binary32 rows 37.5 -> 38.6
  * us); binary32 rows tie rarely and keep the serial one in place. */
 template <int DT>
